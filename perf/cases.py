@@ -1,0 +1,528 @@
+"""Timed cases of the scattering hot path, through the package's public calls.
+
+Ten kinds of call, each at the sizes a user of the package meets:
+
+shell       one q shell of free vectors, as the per-shell loop of the reference's runner does it
+scan        a q scan times one orientation set, coherent, FFT autocorrelation
+xray        the same with one form factor per atom and shell (X-ray)
+static      |A|^2 of one or a few structures (dsp square), the static structure factor
+self        the incoherent function, one FFT autocorrelation per atom and vector
+trajectory  a small trajectory as a whole: staging, factors and its scan
+sphere      multipole average over the sphere
+cylinder    multipole average about an axis
+batch       several uneven trajectories in one call
+network     the control variate's network: training and prediction
+
+Coordinates are random walks (about a site each for "self") at liquid
+density, 0.1 atoms per cubic Angstrom; neutron scattering lengths; q scans
+rounded as the reference's scan builder rounds them.
+"""
+import math
+
+import numpy as np
+import torch
+
+from sassena_amd import Batch, ScatterDevice, synth
+from sassena_amd.mlp import MLP
+
+
+def listed():
+    return [
+        # the reference's own unit of work, one shell of a small protein-sized system: latency
+        {"name": "shell_small", "kind": "shell", "atoms": 1000, "frames": 200, "vectors": 50},
+        # one shell of an ordinary system (the headline trajectory of the benchmark)
+        {"name": "shell", "kind": "shell", "atoms": 20000, "frames": 2000, "vectors": 200},
+        # the benchmark's headline case, a whole scan
+        {"name": "scan", "kind": "scan", "atoms": 20000, "frames": 2000, "shells": 40, "vectors": 200},
+        # X-ray form factors per shell, odd sizes
+        {"name": "xray", "kind": "xray", "atoms": 7001, "frames": 1501, "shells": 21, "vectors": 67},
+        # static structure factor of a single structure
+        {"name": "static", "kind": "static", "atoms": 100000, "frames": 1, "shells": 40, "vectors": 500},
+        # incoherent scattering of a small and of a long trajectory
+        {"name": "self_short", "kind": "self", "atoms": 3000, "frames": 1000, "shells": 8, "vectors": 50},
+        {"name": "self_long", "kind": "self", "atoms": 20000, "frames": 5000, "shells": 3, "vectors": 100},
+        # many small trajectories one after the other through one device
+        {"name": "trajectory", "kind": "trajectory", "atoms": 1000, "frames": 200, "shells": 10, "vectors": 50,
+         "layout": "frames"},
+        # multipole averages of the benchmark's list of moments (l <= 10)
+        {"name": "sphere", "kind": "sphere", "atoms": 20000, "frames": 2000, "shells": 10, "lmax": 10},
+        {"name": "cylinder", "kind": "cylinder", "atoms": 10000, "frames": 2000, "shells": 10, "lmax": 10,
+         "tilted": False},
+        # a set of uneven trajectories in one call
+        {"name": "batch", "kind": "batch", "trajectories": 16, "atoms": 8000, "frames": 2000, "shells": 40,
+         "vectors": 150},
+        # the control variate on 40 shells x 1,000 lags
+        {"name": "network", "kind": "network", "rows": 40000, "steps": 500, "batch": 4096},
+    ]
+
+
+def _log(rng, lo, hi):
+    return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+
+def draw(rng):
+    """A case of the listed kinds with sizes from their whole ranges."""
+    kind = rng.choice(["shell", "scan", "xray", "static", "self", "trajectory", "sphere", "cylinder", "batch",
+                       "network"])
+    if kind == "batch":
+        return {"kind": kind, "trajectories": rng.randint(3, 20), "atoms": _log(rng, 500, 8000),
+                "frames": _log(rng, 100, 2000), "shells": rng.randint(10, 40), "vectors": _log(rng, 20, 150)}
+    if kind == "network":
+        return {"kind": kind, "rows": _log(rng, 1000, 60000), "steps": _log(rng, 50, 500),
+                "batch": _log(rng, 256, 4096)}
+    while True:
+        c = {"kind": kind}
+        if kind == "static":
+            c["atoms"], c["frames"] = _log(rng, 2000, 200000), _log(rng, 1, 24)
+        elif kind == "trajectory":
+            c["atoms"], c["frames"] = _log(rng, 200, 5000), _log(rng, 50, 2000)
+        elif kind == "self":
+            c["atoms"], c["frames"] = _log(rng, 200, 20000), _log(rng, 200, 12000)
+        else:
+            c["atoms"], c["frames"] = _log(rng, 500, 20000), _log(rng, 50, 4000)
+        if kind in ("sphere", "cylinder"):
+            c["shells"], c["lmax"] = rng.randint(1, 12), rng.randint(2, 14)
+            if kind == "cylinder":
+                c["tilted"] = rng.random() < 0.5
+        else:
+            c["shells"] = 1 if kind == "shell" else rng.randint(2, 20) if kind == "self" else rng.randint(4, 60)
+            c["vectors"] = _log(rng, 10, 100 if kind == "self" else 500 if kind == "static" else 300)
+        if kind == "trajectory":
+            c["layout"] = rng.choice(["frames", "atoms", "soa"])
+        most = {"shell": 8e9, "scan": 2e11, "xray": 3e10, "static": 4e9, "self": 3e10, "trajectory": 5e9,
+                "sphere": 4e10, "cylinder": 1e10}[kind]
+        if _terms(c) <= most:
+            return c
+
+
+# ------------------------------------------------------------------ inputs --
+
+def _moments(case):
+    l1 = range(1, case["lmax"] + 1)
+    if case["kind"] == "sphere":
+        return [(0, 0)] + [(l, m) for l in l1 for m in range(-l, l + 1)]
+    return [(0, 0)] + [(l, m) for l in l1 for m in range(4)]
+
+
+def _series(case):
+    """Vectors or moments of a shell."""
+    return len(_moments(case)) if case["kind"] in ("sphere", "cylinder") else case["vectors"]
+
+
+def _terms(case):
+    """(atom, frame, vector or moment) terms of one call."""
+    return case["atoms"] * case["frames"] * case.get("shells", 1) * _series(case)
+
+
+def _generator(seed):
+    return torch.Generator(device="cuda").manual_seed(seed)
+
+
+def _box(atoms):
+    return (atoms / 0.1) ** (1.0 / 3.0)
+
+
+def _walk(g, atoms, frames):
+    """Random walks from uniform starts in the box, sigma 0.1 A per frame: float32 [3][atoms][frames]."""
+    xyz = np.empty((3, atoms, frames), np.float32)
+    for k in range(3):
+        step = 0.1 * torch.randn(atoms, frames, generator=g, device="cuda", dtype=torch.float64)
+        step[:, 0] = _box(atoms) * torch.rand(atoms, generator=g, device="cuda", dtype=torch.float64)
+        xyz[k] = torch.cumsum(step, 1).float().cpu().numpy()
+    del step
+    torch.cuda.empty_cache()
+    return xyz
+
+
+def _bound_walk(g, atoms, frames):
+    """Ornstein-Uhlenbeck walks (std 0.2 A, 50 frames) about uniform sites in the box."""
+    site = _box(atoms) * torch.rand(3, atoms, generator=g, device="cuda", dtype=torch.float64)
+    decay = math.exp(-1.0 / 50.0)
+    kick = 0.2 * math.sqrt(1.0 - decay * decay)
+    out = torch.empty(frames, 3, atoms, device="cuda")
+    pos = 0.2 * torch.randn(3, atoms, generator=g, device="cuda", dtype=torch.float64)
+    for t in range(frames):
+        out[t] = site + pos
+        pos = decay * pos + kick * torch.randn(3, atoms, generator=g, device="cuda", dtype=torch.float64)
+    xyz = out.permute(1, 2, 0).contiguous().cpu().numpy()
+    del out
+    torch.cuda.empty_cache()
+    return xyz
+
+
+def _vectors(case, rng):
+    """|q| of the shells and the unit orientations."""
+    ns = case.get("shells", 1)
+    qlen = synth.linear_shells(0.1, 4.0, ns) if ns > 1 else np.array([rng.uniform(0.3, 2.5)])
+    if case["kind"] == "self":
+        qlen = synth.linear_shells(0.2, 3.0, ns)
+    return qlen, synth.orientations(rng, case["vectors"])
+
+
+def _form_factors(b, qlen):
+    """Gaussian form factors per shell: [shells][atoms]."""
+    z = np.abs(b)
+    return z[None, :] * np.exp(-0.02 * (1.0 + 0.1 * z)[None, :] * np.asarray(qlen)[:, None] ** 2)
+
+
+def _multipole_q(case):
+    q = np.linspace(0.2, 2.0, case["shells"])
+    if case["kind"] == "sphere":
+        return np.stack([0.0 * q, 0.0 * q, q], 1)
+    return np.stack([0.5 * q, 0.0 * q, np.sqrt(0.75) * q], 1)
+
+
+def _axis(case):
+    return (0.3, -0.5, 0.8) if case.get("tilted") else (0.0, 0.0, 1.0)
+
+
+def _trajectory(case, seed):
+    """xyz [3][atoms][frames] and the scattering lengths of a case."""
+    g = _generator(seed)
+    rng = np.random.default_rng(seed)
+    walk = _bound_walk if case["kind"] == "self" else _walk
+    mix = synth.INCOHERENT_MIX if case["kind"] == "self" else synth.COHERENT_MIX
+    return walk(g, case["atoms"], case["frames"]), synth.scattering_lengths(rng, case["atoms"], mix), rng
+
+
+def _member_sizes(case):
+    """The trajectories of a batch: atoms between a tenth of the case's and all of it, uneven in every size."""
+    rng = np.random.default_rng(case["trajectories"])
+    return [{"kind": "scan", "atoms": max(50, int(case["atoms"] * 10 ** rng.uniform(-1, 0))),
+             "frames": max(20, int(case["frames"] * rng.uniform(0.2, 1.0))),
+             "shells": int(rng.integers(max(2, case["shells"] // 4), case["shells"] + 1)),
+             "vectors": int(rng.integers(max(1, case["vectors"] // 4), case["vectors"] + 1))}
+            for _ in range(case["trajectories"])]
+
+
+def _members(case, seed):
+    rng = np.random.default_rng(seed)
+    out = []
+    for one in _member_sizes(case):
+        xyz, b, _ = _trajectory(one, int(rng.integers(1 << 31)))
+        out.append((xyz, b, *_vectors(one, rng)))
+    return out
+
+
+def _rows(case, seed):
+    """Features in the control variate's layout (|q|, lags, correlations, zero padding) and a smooth target."""
+    rng = np.random.default_rng(seed)
+
+    def rows(n):
+        x = np.zeros((n, 16), np.float32)
+        x[:, :3] = rng.random((n, 3))
+        decay = np.exp(-3.0 * x[:, 0] ** 2 * x[:, 2])
+        x[:, 3] = decay * (1.0 + 0.05 * rng.normal(size=n))
+        x[:, 4] = 0.02 * rng.normal(size=n)
+        x[:, 5] = 1.0 + 0.05 * rng.normal(size=n)
+        x[:, 6] = 0.1 * decay * rng.normal(size=n)
+        x[:, 7] = 0.01 * rng.normal(size=n)
+        x[:, 8] = 0.1 * rng.normal(size=n)
+        x[:, 9] = rng.random(n) - 0.5
+        y = 0.8 * x[:, 6] + 0.1 * np.sin(4.0 * x[:, 0]) * (x[:, 3] - x[:, 5]) + 0.01 * rng.normal(size=n)
+        return x, y.astype(np.float32)
+
+    x, y = rows(case["rows"])
+    return x, y, rows(case["rows"])[0]
+
+
+# -------------------------------------------------------------------- calls --
+
+def prepare(case, seed):
+    kind = case["kind"]
+    if kind == "network":
+        x, y, new = _rows(case, seed)
+        net = MLP(seed=seed)
+        return {"case": case, "net": net, "p0": net.params(), "x": x, "y": y, "new": new}
+    if kind == "batch":
+        batch = Batch()
+        batch.stage(_members(case, seed))
+        return {"case": case, "batch": batch}
+    xyz, b, rng = _trajectory(case, seed)
+    dev = ScatterDevice("self" if kind == "self" else "all", "square" if kind == "static" else "autocorrelate")
+    state = {"case": case, "dev": dev}
+    if kind in ("sphere", "cylinder"):
+        state["q"], state["moments"] = _multipole_q(case), np.array(_moments(case), np.int32)
+    else:
+        state["qlen"], state["u"] = _vectors(case, rng)
+        if kind == "shell":
+            state["qv"] = state["qlen"][0] * state["u"]
+        elif kind == "xray":
+            state["b_shell"] = _form_factors(b, state["qlen"])
+    if kind == "trajectory":
+        turn = {"frames": synth.to_frames_aos, "atoms": synth.to_atoms_aos, "soa": lambda a: a}[case["layout"]]
+        state["xyz"], state["b"] = turn(xyz), b
+    else:
+        dev.stage(xyz, layout="soa")
+        dev.set_factors(b)
+    return state
+
+
+def run(state):
+    case = state["case"]
+    kind = case["kind"]
+    if kind == "network":
+        net = state["net"]
+        net.set_params(state["p0"])
+        loss = net.train(state["x"], state["y"], steps=case["steps"], batch=case["batch"])
+        return net.params(), loss, net.predict(state["new"])
+    if kind == "batch":
+        return state["batch"].run()
+    dev = state["dev"]
+    if kind == "shell":
+        return dev.compute_shell(state["qv"])
+    if kind in ("sphere", "cylinder"):
+        return dev.compute_multipole(kind, state["q"], state["moments"], axis=_axis(case))
+    if kind == "xray":
+        return dev.compute_oriented(state["qlen"], state["u"], b_shell=state["b_shell"])
+    if kind == "trajectory":
+        dev.stage(state["xyz"], layout=case["layout"])
+        dev.set_factors(state["b"])
+    return dev.compute_oriented(state["qlen"], state["u"])
+
+
+# --------------------------------------------------------------------- work --
+
+def work(case):
+    """Flops per (atom, frame, vector) term: phase 6, phasor and sums 6; a
+    scan steps the phasor and adds it, 8.  Autocorrelation: 5 L log2 L of the
+    padded length per transform, the back transform once per shell.  Multipole:
+    2 real products and sums per moment, with the Bessel and angular functions
+    by three-term recurrences."""
+    kind = case["kind"]
+    if kind == "network":
+        weights = 16 * 128 + 128 * 128 + 128
+        return {"bytes": 4.0 * (2 * case["rows"] * 17 + 2 * 18817),
+                "flops": 2.0 * weights * (3.0 * case["steps"] * case["batch"] + case["rows"])}
+    if kind == "batch":
+        parts = [work(one) for one in _member_sizes(case)]
+        return {k: sum(p[k] for p in parts) for k in ("bytes", "flops")}
+    na, nf, ns, nv = case["atoms"], case["frames"], case.get("shells", 1), _series(case)
+    fft = 5.0 * 2 * nf * math.log2(2 * nf) if nf > 1 and kind != "static" else 4.0 * nf
+    flops = ns * fft + ns * nv * fft
+    if kind == "self":
+        na = int(round(0.6 * na))
+        flops = ns * fft + ns * nv * na * (fft + 12.0 * nf)
+    elif kind in ("sphere", "cylinder"):
+        lmax = case["lmax"]
+        angular = 3.0 * (lmax + 1) * (lmax + 2) / 2 + 4.0 * lmax if kind == "sphere" else 8.0 * lmax
+        radial = ns * 3.0 * (lmax + 1) * (1 if kind == "sphere" else 2)
+        flops += na * nf * (angular + radial + 2.0 * 2.0 * nv * ns / (2.0 if kind == "sphere" else 1.0))
+    else:
+        flops += (12.0 if kind in ("shell", "xray") else 8.0) * _terms(case)
+    bytes_ = 12.0 * na * nf + 16.0 * ns * nf + (8.0 * ns * na if kind == "xray" else 8.0 * na)
+    return {"bytes": bytes_, "flops": flops}
+
+
+# ----------------------------------------------- the same in 64 bits, plain --
+
+def _correlate(a):
+    """sum over the series a [n][NF] of C(tau) = mean_t conj(a_t) a_{t+tau}, sums of a_m = mean_tau C_m and |a_m|^2."""
+    nf = a.shape[1]
+    x = torch.fft.fft(a, 2 * nf)
+    c = torch.fft.ifft(x.real ** 2 + x.imag ** 2)[:, :nf]
+    c = c / torch.arange(nf, 0, -1, device=a.device, dtype=torch.float64)
+    m = c.mean(1)
+    return c.sum(0), m.sum(), (m.real ** 2 + m.imag ** 2).sum()
+
+
+def _square(a):
+    c = a.real ** 2 + a.imag ** 2
+    m = c.mean(1)
+    return c.sum(0).to(a.dtype), m.sum().to(a.dtype), (m * m).sum()
+
+
+def _results(parts, norm):
+    fqt = torch.stack([p[0] for p in parts]).cpu().numpy() * norm
+    fq = np.array([complex(p[1]) for p in parts]) * norm
+    fq2 = np.array([complex(p[2]) for p in parts]) * norm
+    return fqt, fq, fq2
+
+
+def _exact_shells(xyz, b, qlen, u, reduce, b_shell=None):
+    """Coherent shells: A_sm(t) = sum_j b_j e^{i q_s u_m . r_j(t)}, then reduce over m."""
+    r = torch.from_numpy(xyz).cuda()
+    ns, nm, nf = len(qlen), len(u), xyz.shape[2]
+    amp = torch.empty(ns, nm, nf, dtype=torch.complex128, device="cuda")
+    weights = torch.from_numpy(np.broadcast_to(np.asarray(b), (ns, len(b))) if b_shell is None else b_shell).cuda()
+    d = torch.empty(xyz.shape[1:], dtype=torch.float64, device="cuda")
+    p, f = torch.empty_like(d), torch.empty_like(d)
+    for m in range(nm):
+        d.copy_(r[0]).mul_(float(u[m, 0]))
+        for k in (1, 2):
+            d.add_(f.copy_(r[k]), alpha=float(u[m, k]))
+        for s in range(ns):
+            torch.mul(d, float(qlen[s]), out=p)
+            torch.cos(p, out=f)
+            amp[s, m].real = weights[s] @ f
+            torch.sin(p, out=f)
+            amp[s, m].imag = weights[s] @ f
+    return _results([reduce(amp[s]) for s in range(ns)], 1.0 / nm)
+
+
+def _exact_self(xyz, b, qlen, u):
+    keep = np.flatnonzero(b)
+    r = torch.from_numpy(xyz[:, keep]).cuda().double()
+    w = torch.from_numpy(b[keep]).cuda()[:, None]
+    per = max(1, int(2e7 / xyz.shape[2]))
+    parts = []
+    for q in qlen:
+        total = [0.0, 0.0, 0.0]
+        for v in u:
+            for j in range(0, len(keep), per):
+                p = sum(float(q * v[k]) * r[k, j:j + per] for k in range(3))
+                got = _correlate(torch.polar(w[j:j + per].expand_as(p).contiguous(), p))
+                total = [x + y for x, y in zip(total, got)]
+        parts.append(total)
+    return _results(parts, 1.0 / len(u))
+
+
+def _sph_bessel(L, x):
+    """j_0 .. j_L: upward where x > L, else downward normalised to j_0 or j_1."""
+    x = x.clamp_min(1e-8)
+    s, c = torch.sin(x), torch.cos(x)
+    up = [s / x]
+    up.append((up[0] - c) / x)
+    for n in range(1, L):
+        up.append((2 * n + 1) / x * up[n] - up[n - 1])
+    down = [None] * (L + 1)
+    hi, f = torch.zeros_like(x), torch.full_like(x, 1e-300)
+    for n in range(L + 40 + int(2 * math.sqrt(2 * L)), 0, -1):
+        if n <= L:
+            down[n] = f
+        hi, f = f, (2 * n + 1) / x * f - hi
+        big = f.abs() > 1e200
+        scale = torch.where(big, 1e-200, 1.0)
+        f, hi = f * scale, hi * scale
+        for k in range(n, L + 1):
+            down[k] = down[k] * scale
+    down[0] = f
+    unit = torch.where(up[0].abs() >= up[1].abs(), up[0] / f, up[1] / hi)
+    return [torch.where(x > L, up[n], down[n] * unit) if n > 1 else up[n] for n in range(L + 1)]
+
+
+def _cyl_bessel(N, x):
+    """J_0 .. J_N: upward where x > N, else downward normalised by J_0 + 2 sum J_2k = 1."""
+    x = x.clamp_min(1e-8)
+    up = [torch.special.bessel_j0(x), torch.special.bessel_j1(x)]
+    for n in range(1, N):
+        up.append(2 * n / x * up[n] - up[n - 1])
+    down = [None] * (N + 1)
+    hi, f, norm = torch.zeros_like(x), torch.full_like(x, 1e-300), torch.zeros_like(x)
+    start = N + 40 + int(2 * math.sqrt(2 * N))
+    for n in range(start + start % 2, 0, -1):
+        hi, f = f, 2 * n / x * f - hi
+        if n <= N + 1:
+            down[n - 1] = f
+        if (n - 1) % 2 == 0 and n > 1:
+            norm = norm + 2 * f
+        scale = torch.where(f.abs() > 1e200, 1e-200, 1.0)
+        f, hi, norm = f * scale, hi * scale, norm * scale
+        for k in range(n - 1, N + 1):
+            down[k] = down[k] * scale
+    norm = norm + f
+    return [torch.where(x > N, up[n], down[n] / norm) if n > 1 else up[n] for n in range(N + 1)]
+
+
+def _exact_sphere(xyz, b, q, L, moments):
+    """A_lm = 4 pi i^l sum_j b_j j_l(q r_j) conj(Y_lm), of spherical coordinates rounded to float as they are staged."""
+    na, nf, ns = xyz.shape[1], xyz.shape[2], len(q)
+    amp = torch.zeros(ns, len(moments), nf, dtype=torch.complex128, device="cuda")
+    place = {mo: k for k, mo in enumerate(moments)}
+    per = max(1, int(2e6 / nf))
+    for j in range(0, na, per):
+        x, y, z = torch.from_numpy(xyz[:, j:j + per]).cuda().double()
+        w = torch.from_numpy(b[j:j + per]).cuda()[:, None]
+        r = torch.sqrt(x * x + y * y + z * z)
+        theta = torch.where(r > 0, torch.acos((z / r).clamp(-1, 1)), 0.0).float().double()
+        phi = torch.atan2(y, x)
+        phi = torch.where(phi < 0, phi + 2 * math.pi, phi).float().double()
+        ct, st = torch.cos(theta), torch.sin(theta)
+        radial = [[w * jl for jl in _sph_bessel(L, float(qs) * r.float().double())] for qs in q]
+        pmm = torch.full_like(ct, math.sqrt(1 / (4 * math.pi)))
+        for m in range(L + 1):
+            if m:
+                pmm = -math.sqrt((2 * m + 1) / (2 * m)) * st * pmm
+            c, s = torch.cos(m * phi), torch.sin(m * phi)
+            p0, p1 = torch.zeros_like(pmm), pmm
+            for l in range(m, L + 1):
+                if l > m:
+                    a = math.sqrt((4 * l * l - 1) / (l * l - m * m))
+                    e = math.sqrt(((l - 1) ** 2 - m * m) / (4 * (l - 1) ** 2 - 1)) if l > 1 else 0.0
+                    p0, p1 = p1, a * (ct * p1 - e * p0)
+                yr, yi = p1 * c, p1 * s
+                for k in range(ns):
+                    re, im = (radial[k][l] * yr).sum(0), (radial[k][l] * yi).sum(0)
+                    f = 4 * math.pi * (1j ** l)
+                    amp[k, place[l, m]] += f * torch.complex(re, -im)
+                    if m:
+                        amp[k, place[l, -m]] += f * (-1) ** m * torch.complex(re, im)
+    return _results([_correlate(amp[k]) for k in range(ns)], 1 / (4 * math.pi))
+
+
+def _frame_of(axis):
+    ez = np.asarray(axis, float) / np.linalg.norm(axis)
+    e = np.cross([0.0, 0.0, 1.0], ez)
+    if not np.any(e):
+        e = np.cross([0.0, 1.0, 0.0], ez)
+    er = e / np.linalg.norm(e)
+    return er, np.cross(ez, er), ez
+
+
+def _polar_angle(x, y):
+    """In [0, 2 pi], the half turn added for x < 0 rounded to float as the staged coordinates have it."""
+    half = float(np.float32(math.pi))
+    phi = torch.where(x < 0, torch.atan(y / x) + torch.where(y < 0, -half, half), torch.atan2(y, x))
+    return torch.where(phi < 0, phi + 2 * math.pi, phi)
+
+
+def _exact_cylinder(xyz, b, q, moments, axis):
+    """A_lm = sqrt(2 pi) sum_j b_j e^{i |z_j q_z|} F_lm(r_j q_r, phi_j - phi_q), of cylinder coordinates rounded to
+    float as they are staged."""
+    base = _frame_of(axis)
+    na, nf, ns = xyz.shape[1], xyz.shape[2], len(q)
+    orders = [0 if l == 0 else 2 * l if m < 2 else 2 * l - 1 for l, m in moments]
+    amp = torch.zeros(ns, len(moments), nf, dtype=torch.complex128, device="cuda")
+    per = max(1, int(2e6 / nf))
+    for j in range(0, na, per):
+        p = torch.from_numpy(xyz[:, j:j + per]).cuda().double()
+        w = torch.from_numpy(b[j:j + per]).cuda()[:, None]
+        x, y, z = (sum(float(e[k]) * p[k] for k in range(3)) for e in base)
+        r = torch.sqrt(x * x + y * y).float().double()
+        phi = _polar_angle(x, y).float().double()
+        z = z.float().double()
+        for s in range(ns):
+            qx, qy, qz = (float(np.dot(q[s], e)) for e in base)
+            qphi = float(_polar_angle(torch.tensor(qx).double(), torch.tensor(qy).double()))
+            wave = torch.polar(w.expand_as(z).contiguous(), (z * qz).abs())
+            bessel = _cyl_bessel(max(2, max(orders)), r * math.hypot(qx, qy))
+            for k, (l, m) in enumerate(moments):
+                n = orders[k]
+                if n == 0:
+                    term = wave * bessel[0]
+                else:
+                    ang = torch.cos(n * (phi - qphi)) if m % 2 == 0 else torch.sin(n * (phi - qphi))
+                    f = math.sqrt(2.0) * ((-1) ** l if m < 2 else 1j * (-1) ** (l - 1))
+                    term = f * wave * (bessel[n] * ang)
+                amp[s, k] += math.sqrt(2 * math.pi) * term.sum(0)
+    return _results([_correlate(amp[k]) for k in range(ns)], 1 / (2 * math.pi))
+
+
+def exact(case, seed):
+    kind = case["kind"]
+    if kind == "network":
+        return None
+    if kind == "batch":
+        return [_exact_shells(xyz, b, qlen, u, _correlate) for xyz, b, qlen, u in _members(case, seed)]
+    xyz, b, rng = _trajectory(case, seed)
+    if kind == "sphere":
+        return _exact_sphere(xyz, b, _multipole_q(case)[:, 2], case["lmax"], _moments(case))
+    if kind == "cylinder":
+        return _exact_cylinder(xyz, b, _multipole_q(case), _moments(case), _axis(case))
+    qlen, u = _vectors(case, rng)
+    if kind == "self":
+        return _exact_self(xyz, b, qlen, u)
+    if kind == "shell":
+        return tuple(v[0] for v in _exact_shells(xyz, b, qlen, u, _correlate))
+    return _exact_shells(xyz, b, qlen, u, _square if kind == "static" else _correlate,
+                         _form_factors(b, qlen) if kind == "xray" else None)
