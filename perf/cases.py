@@ -341,22 +341,25 @@ def _results(parts, norm):
 
 def _exact_shells(xyz, b, qlen, u, reduce, b_shell=None):
     """Coherent shells: A_sm(t) = sum_j b_j e^{i q_s u_m . r_j(t)}, then reduce over m."""
-    r = torch.from_numpy(xyz).cuda()
-    ns, nm, nf = len(qlen), len(u), xyz.shape[2]
+    r = torch.from_numpy(xyz).cuda().permute(0, 2, 1).double().contiguous()
+    ns, nm, nf, na = len(qlen), len(u), xyz.shape[2], xyz.shape[1]
     amp = torch.empty(ns, nm, nf, dtype=torch.complex128, device="cuda")
-    weights = torch.from_numpy(np.broadcast_to(np.asarray(b), (ns, len(b))) if b_shell is None else b_shell).cuda()
-    d = torch.empty(xyz.shape[1:], dtype=torch.float64, device="cuda")
+    weights = torch.from_numpy(np.tile(b, (ns, 1)) if b_shell is None else b_shell).cuda()
+    per = max(1, min(nm, int(4e7 / (na * nf))))
+    d = torch.empty(per, nf, na, dtype=torch.float64, device="cuda")
     p, f = torch.empty_like(d), torch.empty_like(d)
-    for m in range(nm):
-        d.copy_(r[0]).mul_(float(u[m, 0]))
-        for k in (1, 2):
-            d.add_(f.copy_(r[k]), alpha=float(u[m, k]))
+    for m in range(0, nm, per):
+        n = min(per, nm - m)
+        for i in range(n):
+            torch.mul(r[0], float(u[m + i, 0]), out=d[i])
+            for k in (1, 2):
+                d[i].add_(r[k], alpha=float(u[m + i, k]))
         for s in range(ns):
             torch.mul(d, float(qlen[s]), out=p)
             torch.cos(p, out=f)
-            amp[s, m].real = weights[s] @ f
+            amp[s, m:m + n].real = (f.view(-1, na) @ weights[s]).view(per, nf)[:n]
             torch.sin(p, out=f)
-            amp[s, m].imag = weights[s] @ f
+            amp[s, m:m + n].imag = (f.view(-1, na) @ weights[s]).view(per, nf)[:n]
     return _results([reduce(amp[s]) for s in range(ns)], 1.0 / nm)
 
 
