@@ -88,11 +88,18 @@ __global__ __launch_bounds__(512) void corr_batch_kernel(const CorrArgs *__restr
     corr_all_block<C, NH, E>(cargs[w.x], w.y, w.z, lds_d);
 }
 
-__global__ __launch_bounds__(256) void final_batch_kernel(const FinalArgs *__restrict__ fargs,
-                                                          const int4 *__restrict__ items) {
-    extern __shared__ double Psh[];
+__global__ __launch_bounds__(kFinalThreads) void final_reduce_batch_kernel(const FinalArgs *__restrict__ fargs,
+                                                                           const int4 *__restrict__ items) {
+    __shared__ double2 sh[kFinalThreads];
     const int4 w = items[blockIdx.x];
-    final_block(fargs[w.x], w.y, w.z, Psh);
+    final_reduce_block(fargs[w.x], w.y, w.z, sh);
+}
+
+__global__ __launch_bounds__(kFinalThreads) void final_transform_batch_kernel(const FinalArgs *__restrict__ fargs,
+                                                                              const int4 *__restrict__ items) {
+    __shared__ double2 sh[kFinalThreads];
+    const int4 w = items[blockIdx.x];
+    final_transform_block(fargs[w.x], w.y, w.z, sh);
 }
 
 using PersistentFn = void (*)(const OrientKernelArgs *, const int4 *, const int *, unsigned *);
@@ -176,9 +183,8 @@ struct Plan {
     // persistent launches in order: tiles of modes 0 / 1, then of mode 2,
     // each by tile shape (largest first)
     std::vector<Queue> queues;
-    int nitems = 0, nfitems = 0;
+    int nitems = 0, nritems = 0, nfitems = 0;
     size_t terms_exact_runs = 0;  // terms of mode-2 tiles stepped without corrections (kind 2)
-    size_t final_lds = 0;
     struct CorrGroup {
         int E, T, first, count;
         size_t lds;
@@ -402,8 +408,7 @@ int build_plan(sx_batch *b, const std::vector<int> &ks, int shape, Plan &P) {
     std::vector<sx::CorrArgs> ca(b->trajs.size());
     std::vector<sx::FinalArgs> fa(b->trajs.size());
     std::map<int, std::vector<int4>> by_len;
-    std::vector<int4> fitems;
-    size_t final_lds = 8;
+    std::vector<int4> ritems, fitems;
     for (int k : ks) {
         const sx_trajectory &t = b->trajs[k];
         TrajWork &tw = b->work[k];
@@ -440,11 +445,15 @@ int build_plan(sx_batch *b, const std::vector<int> &ks, int shape, Plan &P) {
         f.fqt = tw.fqt.as<double>();
         f.fq = tw.fq.as<double>();
         f.fq2 = tw.fq2.as<double>();
-        const int tiles = (int)((t.NF + 255) / 256);
-        for (int s = 0; s < (int)t.nshells; ++s)
-            for (int ti = 0; ti < tiles; ++ti) fitems.push_back(make_int4(k, s, ti, 0));
-        final_lds = std::max(final_lds, sx::final_lds_bytes(c->plan.L));
+        for (int s = 0; s < (int)t.nshells; ++s) {
+            for (int ti = 0; ti < sx::final_reduce_tiles(f); ++ti) ritems.push_back(make_int4(k, s, ti, 0));
+            for (int ti = 0; ti < sx::final_lag_tiles(f); ++ti) fitems.push_back(make_int4(k, s, ti, 0));
+        }
     }
+    // the finalisation's two launches, one list after the other
+    P.nritems = (int)ritems.size();
+    P.nfitems = (int)fitems.size();
+    fitems.insert(fitems.begin(), ritems.begin(), ritems.end());
     std::vector<int4> citems;
     P.groups.clear();
     for (auto &kv : by_len) {
@@ -465,8 +474,6 @@ int build_plan(sx_batch *b, const std::vector<int> &ks, int shape, Plan &P) {
     SXB_HIP(b, P.fitems.ensure(sizeof(int4) * std::max<size_t>(1, fitems.size())));
     if (!fitems.empty())
         SXB_HIP(b, hipMemcpy(P.fitems.p, fitems.data(), sizeof(int4) * fitems.size(), hipMemcpyHostToDevice));
-    P.nfitems = (int)fitems.size();
-    P.final_lds = final_lds;
     return SX_OK;
 }
 
@@ -495,8 +502,11 @@ int launch_rest(sx_batch *b, Plan &P) {
                            P.citems.as<int4>() + g.first);
         SXB_HIP(b, hipGetLastError());
     }
-    hipLaunchKernelGGL(sx::final_batch_kernel, dim3(P.nfitems), dim3(256), P.final_lds, b->stream,
+    hipLaunchKernelGGL(sx::final_reduce_batch_kernel, dim3(P.nritems), dim3(sx::kFinalThreads), 0, b->stream,
                        P.fargs.as<sx::FinalArgs>(), P.fitems.as<int4>());
+    SXB_HIP(b, hipGetLastError());
+    hipLaunchKernelGGL(sx::final_transform_batch_kernel, dim3(P.nfitems), dim3(sx::kFinalThreads), 0, b->stream,
+                       P.fargs.as<sx::FinalArgs>(), P.fitems.as<int4>() + P.nritems);
     SXB_HIP(b, hipGetLastError());
     return SX_OK;
 }
@@ -506,8 +516,6 @@ int capture(sx_batch *b, Plan &P) {
     for (const Plan::CorrGroup &g : P.groups)
         SXB_HIP(b, hipFuncSetAttribute((const void *)sx::corr_batch_fn(g.E),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)g.lds));
-    SXB_HIP(b, hipFuncSetAttribute((const void *)sx::final_batch_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   (int)P.final_lds));
     hipGraph_t g = nullptr;
     SXB_HIP(b, hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
     int rc = launch_amplitude(b, P);

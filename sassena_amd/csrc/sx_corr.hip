@@ -724,24 +724,26 @@ hipError_t launch_weights(const FftPlan &P, int NF, const double2 *tw64, double2
     return hipGetLastError();
 }
 
-// fqt(tau) = R(tau) / (L (NF - tau) NM), R = sum_f P_f e^{+2 pi i f tau / L},
-// P = sum over chunks of the partial power spectra (all FP64); fq and fq2
-// from the per-chunk sums of a and |a|^2 (scaled by 1/NM only, as in
-// all_vectors_scatter_device.cpp:355-360 and self_vectors_scatter_device.cpp:233-238).
-__global__ __launch_bounds__(256) void final_kernel(FinalArgs a) {
-    extern __shared__ double Psh[];
-    final_block(a, blockIdx.y, blockIdx.x, Psh);
+// The back-transform of every shell (final_reduce_block, final_transform_block;
+// fq and fq2 scaled by 1/NM only, as in all_vectors_scatter_device.cpp:355-360
+// and self_vectors_scatter_device.cpp:233-238).
+__global__ __launch_bounds__(kFinalThreads) void final_reduce_kernel(FinalArgs a) {
+    __shared__ double2 sh[kFinalThreads];
+    final_reduce_block(a, blockIdx.y, blockIdx.x, sh);
+}
+
+__global__ __launch_bounds__(kFinalThreads) void final_transform_kernel(FinalArgs a) {
+    __shared__ double2 sh[kFinalThreads];
+    final_transform_block(a, blockIdx.y, blockIdx.x, sh);
 }
 
 hipError_t launch_final(const FinalArgs &a, hipStream_t stream) {
-    const size_t lds = a.ppart ? final_lds_bytes(a.L) : 0;
-    if (lds > 0) {
-        hipError_t e =
-            hipFuncSetAttribute((const void *)final_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-    }
-    const unsigned tiles = a.ppart ? (unsigned)((a.NF + 255) / 256) : 1u;
-    hipLaunchKernelGGL(final_kernel, dim3(tiles, (unsigned)a.nshells), dim3(256), lds, stream, a);
+    hipLaunchKernelGGL(final_reduce_kernel, dim3((unsigned)final_reduce_tiles(a), (unsigned)a.nshells),
+                       dim3(kFinalThreads), 0, stream, a);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess || !a.ppart) return e;
+    hipLaunchKernelGGL(final_transform_kernel, dim3((unsigned)final_lag_tiles(a), (unsigned)a.nshells),
+                       dim3(kFinalThreads), 0, stream, a);
     return hipGetLastError();
 }
 

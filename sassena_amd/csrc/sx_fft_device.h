@@ -937,92 +937,162 @@ struct SelfInputShifted : SelfRows {
     }
 };
 
-// One block of the shell back-transform: shell s, frame tile `tile` (256
-// frames); Psh holds final_lds_bytes(L) of LDS.  fqt(tau) = R(tau) / (L (NF -
-// tau) NM) with R = sum_f P_f e^{+2 pi i f tau / L} in FP64, P the sum of the
-// chunk partials, staged through LDS kFinalChunk bins at a time; tile 0 also
-// writes fq = sum a / NM and fq2 = sum |a|^2 / NM.
-__device__ __forceinline__ void final_block(const FinalArgs &a, int s, int tile, double *Psh) {
-    const int tid = threadIdx.x;
-    if (a.ppart != nullptr) {
-        const double *base = a.ppart + (size_t)s * a.chunks * a.L;
-        const int tau = tile * 256 + tid;
-        const bool live = tau < a.NF;
-        // e^{+2 pi i f tau / L} by repeated products with e^{+2 pi i tau / L},
-        // re-anchored on the FP64 table every 64 bins
-        const long L = a.L;
-        const double2 st = a.tw64[live ? tau : 0];
-        long anchor = 0;  // (f * tau) mod L at the anchors
-        const long jump = (64L * (live ? tau : 0)) % L;
-        double rr0 = 0.0, ri0 = 0.0, rr1 = 0.0, ri1 = 0.0;
-        for (int fc = 0; fc < a.L; fc += kFinalChunk) {
-            const int nc = min(kFinalChunk, a.L - fc);
-            __syncthreads();  // every thread is done with the previous chunk
-            for (int f = tid; f < nc; f += 256) {
-                double acc = 0.0;
-                for (int c = 0; c < a.chunks; ++c) acc += base[(size_t)c * a.L + fc + f];
-                Psh[f] = acc;
-            }
-            __syncthreads();
-            if (live) {
-                for (int f0 = 0; f0 < nc; f0 += 64) {
-                    double2 z = a.tw64[anchor];
-                    anchor += jump;
-                    if (anchor >= L) anchor -= L;
-                    const int f1 = min(f0 + 64, nc);
-                    int f = f0;
-                    for (; f + 1 < f1; f += 2) {
-                        const double p0 = Psh[f], p1 = Psh[f + 1];
-                        rr0 = fma(p0, z.x, rr0);
-                        ri0 = fma(p0, z.y, ri0);
-                        double zr = z.x * st.x - z.y * st.y, zi = z.x * st.y + z.y * st.x;
-                        rr1 = fma(p1, zr, rr1);
-                        ri1 = fma(p1, zi, ri1);
-                        z.x = zr * st.x - zi * st.y;
-                        z.y = zr * st.y + zi * st.x;
-                    }
-                    if (f < f1) {
-                        rr0 = fma(Psh[f], z.x, rr0);
-                        ri0 = fma(Psh[f], z.y, ri0);
-                    }
-                }
-            }
+// The shell back-transform, fqt(tau) = R(tau) / (L (NF - tau) NM) with
+// R = sum_f P_f e^{+2 pi i f tau / L} in FP64, runs as two launches of
+// kFinalThreads-thread blocks:
+//
+// final_reduce_block sums the partials over their chunks, each block 64 bins
+// with its 16 wavefronts on different chunks, in place into the shell's first
+// row; two more blocks per shell sum the chunk sums of a (fq = sum a / NM,
+// fq2 = sum |a|^2 / NM) and the tail lags' partials.
+//
+// final_transform_block forms R for 64 lags, lane = lag, its wavefronts
+// on different sixteenths of the bins.  A lane keeps e^{2 pi i k tau / L} of 16
+// consecutive bins in registers; a group of 16 bins is then 32 FMAs on
+// wave-uniform P (scalar loads) and one complex product with the group's
+// phasor, which steps from group to group and is re-anchored on the FP64
+// table every kFinalAnchor groups: 2.5 FP64 operations a bin and lag.
+//
+// Bound by latency for one shell (too few lags to fill the GPU), else by FP64
+// issue.  The form before it, 256 lags a block that each summed every chunk
+// into LDS and stepped its phasor bin by bin (6 operations), left most CUs
+// idle: 9.76 ms for 3 shells of 10,240 bins x 5,000 lags and about 680 chunks,
+// 0.90 ms for one of 4,096 x 2,000 and 200; both launches together take 63
+// and 16 us.
+constexpr int kFinalThreads = 1024;
+constexpr int kFinalWaves = kFinalThreads / kWave;
+constexpr int kFinalGroup = 16;   // bins a lane holds phasors for
+constexpr int kFinalAnchor = 32;  // groups between two anchors
+
+// Per lane, the sum of x over the block's wavefronts; valid in wavefront 0.
+__device__ __forceinline__ double2 wave_sum2(double2 x, double2 *sh, int wave, int lane) {
+    sh[wave * kWave + lane] = x;
+    __syncthreads();
+    double2 r = make_double2(0.0, 0.0);
+    if (wave == 0)
+        for (int k = 0; k < kFinalWaves; ++k) {
+            const double2 v = sh[k * kWave + lane];
+            r.x += v.x;
+            r.y += v.y;
         }
-        if (live) {
-            const double norm = a.norm != 0.0 ? a.norm : 1.0 / (double)a.NM;
-            double scale = norm / ((double)a.L * (double)(a.NF - tau));
-            double re = (rr0 + rr1) * scale, im = (ri0 + ri1) * scale;
-            if (a.tail && tau >= a.NF - a.tail_k) {
-                // the last lags from the direct FP64 sums
-                const double2 *tp = a.tail + (size_t)s * a.tail_blocks * kTailLags + (a.NF - 1 - tau);
-                double tr = 0.0, ti = 0.0;
-                for (int bb = 0; bb < a.tail_blocks; ++bb) {
-                    tr += tp[(size_t)bb * kTailLags].x;
-                    ti += tp[(size_t)bb * kTailLags].y;
-                }
-                scale = norm / (double)(a.NF - tau);
-                re = tr * scale;
-                im = ti * scale;
-            }
-            a.fqt[((size_t)s * a.NF + tau) * 2] = re;
-            a.fqt[((size_t)s * a.NF + tau) * 2 + 1] = a.conj ? -im : im;
-        }
-    }
-    if (tile == 0 && tid == 0) {
-        double sr = 0.0, si = 0.0, s2 = 0.0;
+    return r;
+}
+
+// Block `tile` of shell s: bins 64 tile .. for tile < final_bin_tiles(a), then
+// one block for a, then (a.tail) one for the tail lags.
+__device__ __forceinline__ void final_reduce_block(const FinalArgs &a, int s, int tile, double2 *sh) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int bins = final_bin_tiles(a);
+    double2 x = make_double2(0.0, 0.0);
+    if (tile < bins) {
+        double *row = a.ppart + (size_t)s * a.chunks * a.L + tile * kWave + lane;
+        double p[4] = {0.0, 0.0, 0.0, 0.0};
+        int c = wave;
+        for (; c + 3 * kFinalWaves < a.chunks; c += 4 * kFinalWaves)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) p[i] += row[(size_t)(c + i * kFinalWaves) * a.L];
+        for (; c < a.chunks; c += kFinalWaves) p[0] += row[(size_t)c * a.L];
+        x.x = (p[0] + p[1]) + (p[2] + p[3]);
+        x = wave_sum2(x, sh, wave, lane);  // every chunk of these bins is read
+        if (wave == 0) row[0] = x.x;
+    } else if (tile == bins) {
         const int na = a.achunks > 0 ? a.achunks : a.chunks;
         const double *ap = a.apart + (size_t)s * na * 4;
-        for (int c = 0; c < na; ++c) {
-            sr += ap[4 * c];
-            si += ap[4 * c + 1];
+        double s2 = 0.0;
+        for (int c = threadIdx.x; c < na; c += kFinalThreads) {
+            x.x += ap[4 * c];
+            x.y += ap[4 * c + 1];
             s2 += ap[4 * c + 2];
         }
-        const double factor = a.norm != 0.0 ? a.norm : 1.0 / (double)a.NM;
-        a.fq[2 * s] = sr * factor;
-        a.fq[2 * s + 1] = (a.conj ? -si : si) * factor;
-        a.fq2[2 * s] = s2 * factor;
-        a.fq2[2 * s + 1] = 0.0;
+        const double2 r = wave_sum2(x, sh, wave, lane);
+        __syncthreads();  // sh is read before it is written again
+        double s2r = wave_sum2(make_double2(s2, 0.0), sh, wave, lane).x;
+        double sr = r.x, si = r.y;
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) {
+            sr += __shfl_xor(sr, off, 64);
+            si += __shfl_xor(si, off, 64);
+            s2r += __shfl_xor(s2r, off, 64);
+        }
+        if (threadIdx.x == 0) {
+            const double factor = a.norm != 0.0 ? a.norm : 1.0 / (double)a.NM;
+            a.fq[2 * s] = sr * factor;
+            a.fq[2 * s + 1] = (a.conj ? -si : si) * factor;
+            a.fq2[2 * s] = s2r * factor;
+            a.fq2[2 * s + 1] = 0.0;
+        }
+    } else {
+        double2 *tp = a.tail + (size_t)s * a.tail_blocks * kTailLags + lane;
+        for (int b = wave; b < a.tail_blocks; b += kFinalWaves) {
+            const double2 v = tp[(size_t)b * kTailLags];
+            x.x += v.x;
+            x.y += v.y;
+        }
+        x = wave_sum2(x, sh, wave, lane);
+        if (wave == 0) tp[0] = x;
     }
+}
+
+// Lags 64 tile .. of shell s, from the rows that final_reduce_block left.
+__device__ __forceinline__ void final_transform_block(const FinalArgs &a, int s, int tile, double2 *sh) {
+    static_assert(kTailLags == kWave, "one lane a tail lag");
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int tau = tile * kWave + lane;
+    const unsigned L = (unsigned)a.L, t = (unsigned)min(tau, a.NF - 1);  // t < L / 2
+    const auto P = (const __attribute__((address_space(4))) double *)(a.ppart + (size_t)s * a.chunks * a.L);
+    // e^{2 pi i k t / L} of a group's bins, and the step from group to group
+    double wr[kFinalGroup], wi[kFinalGroup];
+    unsigned e = 0;
+#pragma unroll
+    for (int k = 0; k < kFinalGroup; ++k) {
+        const double2 z = a.tw64[e];
+        wr[k] = z.x;
+        wi[k] = z.y;
+        e += t;
+        if (e >= L) e -= L;
+    }
+    const double2 st = a.tw64[e];  // e = kFinalGroup t mod L
+    // L is a multiple of 512: equal runs of L / 256 groups a wavefront
+    const int ngroups = (int)(L / (kFinalGroup * kFinalWaves));
+    int g = wave * ngroups;
+    const int gend = g + ngroups;
+    unsigned anchor = (L / kFinalWaves) * (((unsigned)wave * t) % kFinalWaves);
+    const unsigned jump = (unsigned)(((unsigned long long)(kFinalGroup * kFinalAnchor) * t) % L);
+    double rr = 0.0, ri = 0.0;
+    while (g < gend) {
+        double2 z = a.tw64[anchor];
+        anchor += jump;
+        if (anchor >= L) anchor -= L;
+        const int ge = min(g + kFinalAnchor, gend);
+        for (; g < ge; ++g) {
+            double sr = 0.0, si = 0.0;
+#pragma unroll
+            for (int k = 0; k < kFinalGroup; ++k) {
+                const double p = P[g * kFinalGroup + k];
+                sr = fma(p, wr[k], sr);
+                si = fma(p, wi[k], si);
+            }
+            rr = fma(z.x, sr, fma(-z.y, si, rr));
+            ri = fma(z.x, si, fma(z.y, sr, ri));
+            const double zr = z.x * st.x - z.y * st.y;
+            z.y = z.x * st.y + z.y * st.x;
+            z.x = zr;
+        }
+    }
+    const double2 R = wave_sum2(make_double2(rr, ri), sh, wave, lane);
+    if (wave != 0 || tau >= a.NF) return;
+    const double norm = a.norm != 0.0 ? a.norm : 1.0 / (double)a.NM;
+    double scale = norm / ((double)a.L * (double)(a.NF - tau));
+    double re = R.x * scale, im = R.y * scale;
+    if (a.tail && tau >= a.NF - a.tail_k) {
+        // the last lags from the direct FP64 sums
+        const double2 v = a.tail[(size_t)s * a.tail_blocks * kTailLags + (a.NF - 1 - tau)];
+        scale = norm / (double)(a.NF - tau);
+        re = v.x * scale;
+        im = v.y * scale;
+    }
+    a.fqt[((size_t)s * a.NF + tau) * 2] = re;
+    a.fqt[((size_t)s * a.NF + tau) * 2 + 1] = a.conj ? -im : im;
 }
 
 // ------------------------------------------------- series of N1 > 1 rows ---

@@ -235,19 +235,22 @@ struct FinalArgs {
     int achunks = 0;       // entries of apart per shell (0: chunks)
     // "self": the last tail_k lags summed directly in FP64 (tail[shell][tail_blocks][tail_k],
     // entry k = lag NF-1-k) replace the transform's values there
-    const double2 *tail = nullptr;
+    double2 *tail = nullptr;
     int tail_k = 0, tail_blocks = 0;
     double norm = 0.0;     // final factor (1/NM for vector averages); 0 means 1/NM
-    const double *ppart;   // nullptr: fqt already written by the series kernel
+    double *ppart;         // summed in place into the first chunk's row; nullptr: fqt already
+                           // written by the series kernel
     const double *apart;
     const double2 *tw64;   // [L] exp(+2 pi i e / L), double
     int conj;              // 1 for the direct method (conjugate result)
     double *fqt, *fq, *fq2;
 };
 hipError_t launch_final(const FinalArgs &a, hipStream_t stream);
-// Bins of the summed power spectrum one block of final_kernel holds in LDS at a time.
-constexpr int kFinalChunk = 8192;
-inline size_t final_lds_bytes(int L) { return sizeof(double) * (size_t)(L < kFinalChunk ? L : kFinalChunk); }
+// Blocks per shell of its two launches: 64 bins each, one for a and one for
+// the tail lags where there are any; then 64 lags each.
+__host__ __device__ inline int final_bin_tiles(const FinalArgs &a) { return a.ppart ? (a.L + kWave - 1) / kWave : 0; }
+inline int final_reduce_tiles(const FinalArgs &a) { return final_bin_tiles(a) + 1 + (a.tail ? 1 : 0); }
+inline int final_lag_tiles(const FinalArgs &a) { return (a.NF + kWave - 1) / kWave; }
 
 // dsp.type square (mode 1) / plain (mode 2) on coherent amplitudes; norm is
 // the final factor of fqt (1/NM for vector averages)
