@@ -77,11 +77,12 @@ typedef struct sx_config {
                             (cylinder, 12 B) coordinates of every (atom, frame) 1 formed once
                             per call in a pre-pass, 2 formed by the amplitude kernel itself;
                             0 picks 1 up to 16 GB of terms, else 2.  With 0 and 1 the Bessel
-                            functions of every (shell, atom, frame) also come from a pre-pass
-                            (8 B each; sphere j_0..j_lmax for lmax <= 16, cylinder J_0..J_nmax for
-                            orders nmax <= 32) while the table stays within 96 GB and leaves
-                            4 GB of device memory free; 3 is 1 without that table (the two
-                            lowest only, the rest by recurrence in the kernel) */
+                            functions of every (shell, atom, frame) are formed once per call:
+                            sphere, degrees up to 16, inside a kernel that sums products of
+                            radial and angular factors; cylinder, orders up to 32, in a
+                            pre-pass (8 B each) while that table stays within 96 GB and leaves
+                            4 GB of device memory free; 3 is 1 without these (the two lowest
+                            only, the rest by recurrence in the kernel) */
     int reserved[6];
 } sx_config;
 

@@ -130,8 +130,9 @@ int pick_split(const sx_ctx *c, int V, int vb) {
 constexpr size_t kSplitAmpBudget = (size_t)4 << 30;
 // Largest buffer of per-(atom, frame) spherical terms of the sphere multipole path.
 constexpr size_t kSphereTermBudget = (size_t)16 << 30;
-// The sphere's table of j_l per (shell, degree, atom, frame): at most this
-// much, and only while this much device memory stays free beside it.
+// The cylinder's table of J_n per (shell, order, atom, frame) and the sphere's
+// partial sums: at most this much, and only while this much device memory
+// stays free beside it.
 constexpr size_t kBesselTableBudget = (size_t)96 << 30;
 constexpr size_t kBesselTableMargin = (size_t)4 << 30;
 
@@ -155,18 +156,19 @@ int round_filling_split(long base, int first, long resident, size_t NAp, size_t 
     return split;
 }
 
-// Whether the sphere's Bessel table of `bytes` may be held: within its
-// budget, and with kBesselTableMargin of device memory left beside it.
-bool bessel_table_fits(sx_ctx *c, size_t bytes) {
+// Whether `buf` may hold `bytes`: within the budget, and with
+// kBesselTableMargin of device memory left beside it.
+bool multipole_buffer_fits(const DevBuf &buf, size_t bytes) {
     if (bytes > kBesselTableBudget) return false;
-    if (c->mpjt.p && bytes <= c->mpjt.cap) return true;
+    if (buf.p && bytes <= buf.cap) return true;
     size_t fr = 0, tot = 0;
     if (hipMemGetInfo(&fr, &tot) != hipSuccess) return false;
-    return fr + c->mpjt.cap >= bytes + kBesselTableMargin;
+    return fr + buf.cap >= bytes + kBesselTableMargin;
 }
 
-// Atom ranges of the multipole kernel.  Its workgroups each sum every atom of
-// their range for one (frame tile, shell, group of 4 moment blocks): the rule
+// Atom ranges of a multipole call, each of which rounds its amplitudes to
+// FP32 once.  The workgroups of multipole_kernel each sum every atom of their
+// range for one (frame tile, shell, group of 4 moment blocks): the rule
 // above, then the split that fills whole rounds of resident workgroups.
 int pick_multipole_split(sx_ctx *c, int kind, int ns, int nmo, int *split) {
     const long base = sx::multipole_base_blocks(c->NFp, ns, nmo, kind);
@@ -521,6 +523,7 @@ int run_batch(sx_ctx *c, int ns, size_t NM, const double *qv, const double *qlen
             const size_t sph_bytes =
                 (mp->kind == 0 ? sx::kSphereTermBytes : sx::kCylinderTermBytes) * c->NAp * c->NFp;
             const int terms = c->cfg.multipole_terms;
+            bool summed = false;  // the amplitudes are there
             if (terms == 1 || terms == 3 || (terms == 0 && sph_bytes <= kSphereTermBudget)) {
                 SX_HIP(c, c->mpsph.ensure(sph_bytes));
                 if (mp->kind == 0)
@@ -528,37 +531,59 @@ int run_batch(sx_ctx *c, int ns, size_t NM, const double *qv, const double *qlen
                 else
                     SX_HIP(c, sx::launch_multipole_cylinder_terms(ma, c->mpsph.p, c->stream));
                 ma.sph = c->mpsph.p;
-                // sphere up to degree 16, cylinder up to order 32: every
-                // Bessel function of every (shell, atom, frame) once per call
-                // when the table fits; else the two lowest (16 B each) within
-                // the terms' budget
-                int L1 = mp->plm_l1;
+                // sphere, degrees up to 16: sums of products of radial and
+                // angular factors
+                sx::SpherePlan sp;
+                int sub = 0;
+                if (mp->kind == 0 && terms != 3 && sx::sphere_sums_grid_fits(ns, split) &&
+                    *std::max_element(mp->qinfo.begin(), mp->qinfo.end()) * c->rmax < 0.99 * sx::kSphereMaxArg &&
+                    sx::make_sphere_plan(mp->moments.data(), (int)NM, ns, &sp)) {
+                    int cus = 0;
+                    SX_HIP(c, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->cfg.device));
+                    sub = sx::sphere_parts_per_range(sp, c->NFp, c->NAp, split, std::max(cus, 1));
+                    while (sub > 0 &&
+                           !multipole_buffer_fits(c->mpsum, sx::sphere_parts_bytes(sp, c->NFp, ns, split, sub)))
+                        sub /= 2;
+                }
+                // cylinder up to order 32: every Bessel function of every
+                // (shell, atom, frame) once per call when the table fits; else
+                // (and for the sphere above degree 16) the two lowest (16 B
+                // each) within the terms' budget
+                int N1 = 1;
                 if (mp->kind == 1) {
-                    L1 = 1;
                     for (size_t k = 0; k + 1 < mp->moments.size(); k += 2) {
                         const int l = mp->moments[k], m = mp->moments[k + 1];
                         const int n = (l == 0 || m > 3 || m < 0) ? 0 : (m <= 1 ? 2 * l : 2 * l - 1);
-                        L1 = std::max(L1, n + 1);
+                        N1 = std::max(N1, n + 1);
                     }
                 }
-                const int L1max = mp->kind == 0 ? sx::kBesselTableL1 : sx::kCylTableN1;
-                // (the cylinder's table also holds two phases per (shell, atom, frame))
-                const size_t tab_bytes = (sizeof(double) * (size_t)std::max(L1, 1) +
-                                          (mp->kind == 1 ? 2 * sizeof(double2) : 0)) *
-                                         (size_t)ns * c->NAp * c->NFp;
+                // (the table also holds two phases per (shell, atom, frame))
+                const size_t tab_bytes =
+                    (sizeof(double) * (size_t)N1 + 2 * sizeof(double2)) * (size_t)ns * c->NAp * c->NFp;
                 const size_t j01_bytes = sizeof(double2) * (size_t)ns * c->NAp * c->NFp;
-                if (terms != 3 && L1 >= 1 && L1 <= L1max && bessel_table_fits(c, tab_bytes)) {
+                if (sub > 0) {
+                    std::vector<char> tables(sx::sphere_table_bytes(sp));
+                    sx::sphere_tables(sp, tables.data());
+                    SX_HIP(c, c->mptab.ensure(tables.size()));
+                    SX_HIP(c, hipMemcpyAsync(c->mptab.p, tables.data(), tables.size(), hipMemcpyHostToDevice,
+                                             c->stream));
+                    SX_HIP(c, c->mpsum.ensure(sx::sphere_parts_bytes(sp, c->NFp, ns, split, sub)));
+                    SX_HIP(c, sx::launch_sphere_sums(ma, sp, c->mptab.p, sub, c->mpsum.p, c->stream));
+                    summed = true;
+                } else if (mp->kind == 1 && terms != 3 && N1 <= sx::kCylTableN1 &&
+                           multipole_buffer_fits(c->mpjt, tab_bytes)) {
                     SX_HIP(c, c->mpjt.ensure(tab_bytes));
-                    SX_HIP(c, sx::launch_multipole_bessel_table(ma, L1, c->mpjt.p, c->stream));
+                    SX_HIP(c, sx::launch_multipole_bessel_table(ma, N1, c->mpjt.p, c->stream));
                     ma.jtab = c->mpjt.p;
-                    ma.jl1 = L1;
+                    ma.jl1 = N1;
                 } else if (j01_bytes <= kSphereTermBudget) {
                     SX_HIP(c, c->mpj.ensure(j01_bytes));
                     SX_HIP(c, sx::launch_multipole_bessel01(ma, c->mpj.p, c->stream));
                     ma.cj01 = c->mpj.p;
                 }
             }
-            SX_HIP(c, sx::launch_multipole(ma, c->stream));
+            if (!summed)
+                SX_HIP(c, sx::launch_multipole(ma, c->stream));
         } else if (oriented) {
             const sx::OrientArgs oa = oriented_args(c, ns, (int)NM, bptr, b_shell != nullptr, shape, split);
             int plain = 0;
@@ -856,7 +881,7 @@ void sx_destroy(sx_ctx *c) {
     if (!c) return;
     (void)hipSetDevice(c->cfg.device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
-    for (DevBuf *d : {&c->coords, &c->b, &c->twL, &c->twL64, &c->twp, &c->twp64, &c->tw64, &c->w, &c->aidx, &c->apair, &c->tail, &c->qrev, &c->qlen, &c->uvec, &c->brow, &c->bshell, &c->mpmom, &c->mpq, &c->mpsph, &c->mpj, &c->mpjt, &c->qres, &c->redbuf, &c->amp,
+    for (DevBuf *d : {&c->coords, &c->b, &c->twL, &c->twL64, &c->twp, &c->twp64, &c->tw64, &c->w, &c->aidx, &c->apair, &c->tail, &c->qrev, &c->qlen, &c->uvec, &c->brow, &c->bshell, &c->mpmom, &c->mpq, &c->mpsph, &c->mpj, &c->mpjt, &c->mptab, &c->mpsum, &c->qres, &c->redbuf, &c->amp,
                       &c->ppart, &c->apart, &c->fqt, &c->fq, &c->fq2, &c->stage, &c->stage2})
         d->release();
     for (auto &e : c->ev)

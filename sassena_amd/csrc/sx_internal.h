@@ -283,21 +283,54 @@ struct MultipoleArgs {
     // (cylinder) per (shell, atom, frame) from launch_multipole_bessel01, or
     // nullptr to form them in the kernel
     const void *cj01 = nullptr;
-    // sphere: j_l for l < jl1 per (shell, degree, atom, frame) from
+    // cylinder: J_n for n < jl1 per (shell, order, atom, frame) from
     // launch_multipole_bessel_table, or nullptr
     const void *jtab = nullptr;
     int jl1 = 0;
 };
+// The sphere average as sums of products of radial and angular factors, for
+// moment lists of degrees below kSphereSumL1 and arguments |q| r up to
+// kSphereMaxArg: its schedule and tables (host), and the launch, from the
+// sphere terms (m.sph).  Each atom range is summed in `sub` parts in FP64
+// (parts, sphere_parts_bytes), which are added before the amplitude of the
+// range is rounded to FP32.
+constexpr int kSphereSumL1 = 17;
+constexpr double kSphereMaxArg = 1e5;
+// What a wavefront does for one degree l of two orders m, m + 1 (m even).
+struct SphereEntry {
+    double alpha1, alpha2;  // recurrence coefficients of the two orders at l
+    int l;
+    int skip;               // steps from degree m to l without sums, or -1: l follows the entry before
+    int first;              // alpha[m][m]
+    int f1, f2;             // powers of u of the two orders
+    int pair;               // where the sums go, or -1: unused
+};
+struct SpherePlan {
+    int L1 = 0, M1 = 0;        // degrees, orders
+    int nd = 0;                // (pair of orders, degree) entries
+    int kernel = -1, groups = 0, CA = 0;
+    std::vector<SphereEntry> sched;  // per wavefront, its entries
+    std::vector<double> alpha; // [M1 + 1][L1] coefficients of the recurrence in the degree
+    std::vector<double> scale; // [nmo] normalisation of the finished sums
+    std::vector<int2> entry;   // [nmo] where each moment's sums are, and its phase
+};
+inline bool sphere_sums_grid_fits(int ns, int split) { return (size_t)ns * split <= 65535; }
+bool make_sphere_plan(const int *moments, int nmo, int ns, SpherePlan *plan);
+int sphere_parts_per_range(const SpherePlan &p, size_t NFp, size_t NAp, int split, int cus);
+size_t sphere_parts_bytes(const SpherePlan &p, size_t NFp, int ns, int split, int sub);
+size_t sphere_table_bytes(const SpherePlan &p);
+void sphere_tables(const SpherePlan &p, void *out);  // host buffer of sphere_table_bytes
+hipError_t launch_sphere_sums(const MultipoleArgs &m, const SpherePlan &p, const void *tables, int sub, void *parts,
+                              hipStream_t stream);
+
 hipError_t launch_multipole(const MultipoleArgs &m, hipStream_t stream);
-// Degrees the sphere's Bessel table holds at most (l <= 16), and orders the
-// cylinder's (n <= 32, the orders 2l and 2l - 1 of l <= 16).
-constexpr int kBesselTableL1 = 17;
+// Orders the cylinder's Bessel table holds at most (n <= 32, the orders 2l
+// and 2l - 1 of l <= 16).
 constexpr int kCylTableN1 = 33;
-// j_0 .. j_{L1-1} (sphere) or J_0 .. J_{L1-1} (cylinder) of every (shell,
-// atom, frame) of a call from its terms (m.sph), into
-// out[(s L1 + l) NAp NFp + atom NFp + frame] (FP64); the cylinder's table
-// then holds (cos, sin) of sgn z q_z and of phi - q_phi per (shell, 2, atom,
-// frame) as double2 (32 B per (shell, atom, frame) more).
+// J_0 .. J_{L1-1} of every (shell, atom, frame) of a cylinder call from its
+// terms (m.sph), into out[(s L1 + n) NAp NFp + atom NFp + frame] (FP64), then
+// (cos, sin) of sgn z q_z and of phi - q_phi per (shell, 2, atom, frame) as
+// double2 (32 B per (shell, atom, frame) more).
 hipError_t launch_multipole_bessel_table(const MultipoleArgs &m, int L1, void *out, hipStream_t stream);
 // Workgroups of the multipole kernel that fit one CU, and its workgroups per
 // atom range (kind 0, sphere: kSphereShells shells per workgroup).
