@@ -303,6 +303,10 @@ OrientKernelArgs make_orient_args(const OrientArgs &a) {
     k.q0 = a.q0;
     k.qres = a.qres;
     k.lines = a.ap == 2 ? a.lines : nullptr;
+    k.pack = nullptr;
+    k.parts = nullptr;
+    k.sub = 1;
+    k.NF = 0;
     return k;
 }
 
@@ -416,6 +420,136 @@ hipError_t launch_amp_oriented(const OrientArgs &a, hipStream_t stream) {
         case 3: return launch_oriented_shape<1, 16>(k, per_row, blocks, stream);
         default: return launch_oriented_shape<1, 20>(k, per_row, blocks, stream);
     }
+}
+
+// ------------------------------------------------------- few frames ------
+
+// pack[t][j] = (x, y, z, b) of atom j at frame t < NF; padding atoms as staged.
+__global__ __launch_bounds__(256) void pack_frames_kernel(const float *__restrict__ X, const float *__restrict__ Y,
+                                                          const float *__restrict__ Z, const float *__restrict__ b,
+                                                          size_t NAp, size_t NFp, float4 *__restrict__ pack) {
+    const size_t j = (size_t)blockIdx.x * 256 + threadIdx.x, t = blockIdx.y;
+    if (j >= NAp) return;
+    const size_t e = j * NFp + t;
+    pack[t * NAp + j] = make_float4(X[e], Y[e], Z[e], b[j]);
+}
+
+// Work of a wavefront of the few-frames launch, items in the order
+// (frame, range, part, shell tile, orientation group), the last fastest, so that the
+// wavefronts of a CU read the same atoms.
+struct FewItem {
+    int t, sp, part, sg, og;
+};
+
+__device__ __forceinline__ bool few_item(const OrientKernelArgs &a, FewItem &w) {
+    int i = __builtin_amdgcn_readfirstlane((int)blockIdx.x * 4 + (int)(threadIdx.x >> 6));
+    w.og = i % a.ogroups;
+    i /= a.ogroups;
+    w.sg = i % a.sgroups;
+    i /= a.sgroups;
+    w.part = i % a.sub;
+    i /= a.sub;
+    w.sp = i % a.split;
+    w.t = i / a.split;
+    return w.t < a.NF;
+}
+
+template <int VS, bool PER_ROW_B>
+__global__ __launch_bounds__(256, 2) void amp_few_kernel(OrientKernelArgs a) {
+    FewItem w;
+    if (!few_item(a, w)) return;
+    oriented_tile<1, VS, PER_ROW_B, true, true>(a, w.t, w.sp, w.og, w.sg * VS, w.part);
+}
+
+template <int VS>
+__global__ __launch_bounds__(256, 2) void amp_few_res_kernel(OrientKernelArgs a) {
+    extern __shared__ double tot_lds[];
+    FewItem w;
+    if (!few_item(a, w)) return;
+    residual_tile<1, VS, true>(a, w.t, w.sp, w.og, w.sg * VS, tot_lds, w.part);
+}
+
+// amp[v][t] = the ranges' amplitudes, each rounded to FP32 from the FP64 sum
+// of its parts, added in FP32 in the ranges' order.
+__global__ __launch_bounds__(kWave) void few_amplitudes_kernel(const double2 *__restrict__ parts, int split, int sub,
+                                                             int V, int NF, size_t NFp, float2 *__restrict__ amp) {
+    const size_t i = (size_t)blockIdx.x * kWave + threadIdx.x, n = (size_t)V * NF;
+    if (i >= n) return;
+    float2 s = make_float2(0.f, 0.f);
+    for (int k = 0; k < split; ++k) {
+        double2 v = make_double2(0.0, 0.0);
+#pragma unroll 8
+        for (int p = 0; p < sub; ++p) {
+            const double2 x = parts[((size_t)k * sub + p) * n + i];
+            v.x += x.x;
+            v.y += x.y;
+        }
+        const float re = (float)v.x, im = (float)v.y;
+        s.x = k ? s.x + re : re;
+        s.y = k ? s.y + im : im;
+    }
+    amp[(i / NF) * NFp + i % NF] = s;
+}
+
+// Lane = orientation pays where the frames' padding (NFp lanes for NF frames)
+// exceeds that of the orientations by a third: one frame of 100,000 atoms, 40
+// shells x 500 orientations: 18.4 ms with lane = frame, 0.47 ms so (packing and
+// adding the parts 0.03 ms more), bound by instruction issue as the other form
+// is.  Up to that third the other form's coalesced coordinates need no packing.
+bool few_frames(size_t NF, size_t NFp, int NM) {
+    const double lanes = (double)NF * ((NM + kWave - 1) / kWave * kWave);
+    return NFp == (size_t)kWave && lanes * 4.0 / 3.0 <= (double)NFp * NM;
+}
+
+// Parts of an atom range, of at least 4 folds: about 4096 wavefronts in all.
+int few_parts(size_t NF, size_t NAp, int NM, int ns, int split, int shape) {
+    const long items = (long)NF * split * ((NM + kWave - 1) / kWave) * ((ns + kShapeVS[shape] - 1) / kShapeVS[shape]);
+    const long most = std::max<long>(1, (long)(NAp / split / 256));
+    return (int)std::max<long>(1, std::min(most, 4096 / std::max<long>(items, 1)));
+}
+
+template <int VS>
+static hipError_t launch_few_shape(const OrientKernelArgs &k, bool per_row, unsigned blocks, hipStream_t stream) {
+    if (k.ap == 2) {
+        if (per_row) return hipErrorInvalidValue;
+        const void *fn = (const void *)amp_few_res_kernel<VS>;
+        const size_t lds = kResidualLds<1, VS>;
+        hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return e;
+        hipLaunchKernelGGL((amp_few_res_kernel<VS>), dim3(blocks), dim3(256), lds, stream, k);
+    } else if (per_row)
+        hipLaunchKernelGGL((amp_few_kernel<VS, true>), dim3(blocks), dim3(256), 0, stream, k);
+    else
+        hipLaunchKernelGGL((amp_few_kernel<VS, false>), dim3(blocks), dim3(256), 0, stream, k);
+    return hipGetLastError();
+}
+
+hipError_t launch_amp_few(const OrientArgs &a, int NF, int sub, float4 *pack, double2 *parts, hipStream_t stream) {
+    if (a.shape < 0 || a.shape >= kOrientShapes || sub < 1 || NF < 1 || (size_t)NF > a.NFp) return hipErrorInvalidValue;
+    OrientKernelArgs k = make_orient_args(a);
+    k.ogroups = (a.NM + kWave - 1) / kWave;
+    k.pack = pack;
+    k.parts = parts;
+    k.sub = sub;
+    k.NF = NF;
+    hipLaunchKernelGGL(pack_frames_kernel, dim3((unsigned)((a.NAp + 255) / 256), (unsigned)NF), dim3(256), 0, stream,
+                       k.X, k.Y, k.Z, a.b, a.NAp, a.NFp, pack);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    const size_t items = (size_t)NF * a.split * sub * k.sgroups * k.ogroups;
+    if (items > (size_t)1 << 30) return hipErrorInvalidValue;
+    const unsigned blocks = (unsigned)((items + 3) / 4);
+    const bool per_row = a.per_shell_b != 0;
+    switch (kShapeVS[a.shape]) {
+        case 4: e = launch_few_shape<4>(k, per_row, blocks, stream); break;
+        case 8: e = launch_few_shape<8>(k, per_row, blocks, stream); break;
+        case 16: e = launch_few_shape<16>(k, per_row, blocks, stream); break;
+        default: e = launch_few_shape<20>(k, per_row, blocks, stream); break;
+    }
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(few_amplitudes_kernel, dim3((unsigned)(((size_t)k.V * NF + kWave - 1) / kWave)), dim3(kWave), 0,
+                       stream, parts, a.split, sub, k.V, NF, a.NFp, a.amp);
+    return hipGetLastError();
 }
 
 template <int VM, int VS>

@@ -25,6 +25,12 @@ struct OrientKernelArgs {
     double q0;             // |q_0| / 2 pi of the ideal grid (ap == 2)
     const float *qres;     // [ns] residuals of the shells against the ideal grid (ap == 2)
     const TileLine *lines; // [ns] lines of the tiles at their first shells (ap == 2)
+    // Few frames (lane = orientation, oriented_tile_body with LQ): the atoms
+    // of a frame packed with their factors, [NF][NAp] (x, y, z, b), and the FP64
+    // sums of every part of an atom range, [split * sub][V][NF]
+    const float4 *pack;
+    double2 *parts;
+    int sub, NF;
 };
 
 // Workgroup LDS of the residual-corrected tile: the FP64 totals of the 4
@@ -54,6 +60,13 @@ OrientKernelArgs make_orient_args(const OrientArgs &a);
 //
 // Atom sums run in FP32 over sub-chunks of CH atoms (coordinates loaded
 // together) and are folded into FP64 totals every kFold atoms.
+//
+// LQ: the tile of a trajectory of few frames, where lanes of one frame each
+// would mostly be padding.  Lane = orientation: frame `ft`, orientations 64 og +
+// lane, the coordinates wave-uniform (scalar loads of the packed atoms);
+// `part` of a.sub whole-fold parts of the atom range, whose FP64 totals go to
+// a.parts.  Every amplitude goes through the same operations on the same
+// groups of atoms in both forms.
 
 // Wave-uniform, read-only kernel data (orientations, shells, residuals,
 // scattering factors) seen through the constant address space, so that it is
@@ -73,20 +86,21 @@ __device__ __forceinline__ int tile_flags(const OrientKernelArgs &a, int sbase) 
     return uniform_ptr(a.lines)[sbase].flags;
 }
 
-template <int VM, int VS, bool PER_ROW_B, int MODE, bool BUF>
+template <int VM, int VS, bool PER_ROW_B, int MODE, bool BUF, bool LQ = false>
 __device__ __forceinline__ void oriented_tile_body(const OrientKernelArgs &a, int ft, int sp, int og, int sbase,
-                                                   double *__restrict__ tot) {
+                                                   double *__restrict__ tot, int part = 0) {
     constexpr bool AP = MODE >= 1;
     constexpr bool LT = MODE >= 2;  // FP64 totals in LDS, the tile's own line
     constexpr bool UPC = MODE == 2 || MODE == 4, DNC = MODE == 2 || MODE == 5;
     constexpr bool RES = UPC || DNC;
     static_assert(!(LT && PER_ROW_B), "residual-corrected tiles take one factor per atom");
-    constexpr int CH = 16;     // atoms per coordinate batch
+    static_assert(!LQ || VM == 1, "one orientation a lane");
+    constexpr int CH = LQ ? 8 : 16;  // atoms per coordinate batch
     constexpr int kFold = 64;  // atoms per FP32 partial sum
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
-    const int mbase = (og * 4 + wave) * VM;
-    const size_t t = (size_t)ft * kWave + lane;
+    const int mbase = LQ ? og * kWave + lane : (og * 4 + wave) * VM;
+    const size_t t = LQ ? (size_t)ft : (size_t)ft * kWave + lane;
 
     const auto U = uniform_ptr(a.u);
     const auto QL = uniform_ptr(a.qlen);
@@ -132,8 +146,13 @@ __device__ __forceinline__ void oriented_tile_body(const OrientKernelArgs &a, in
             }
         }
 
-    const size_t j0 = (size_t)sp * a.atoms_per_split;
-    const size_t j1 = min(a.natoms, j0 + (size_t)a.atoms_per_split);
+    size_t j0 = (size_t)sp * a.atoms_per_split;
+    size_t j1 = min(a.natoms, j0 + (size_t)a.atoms_per_split);
+    if constexpr (LQ) {
+        const size_t folds = j1 > j0 ? (j1 - j0 + kFold - 1) / kFold : 0;
+        j1 = min(j1, j0 + folds * (part + 1) / a.sub * kFold);
+        j0 += folds * part / a.sub * kFold;
+    }
     // BUF: coordinates through buffer loads, a wave-uniform resource per
     // coordinate batch (base = first atom of the batch, this frame tile), the
     // atom's row as the scalar offset and the lane's frame as the vector
@@ -159,7 +178,17 @@ __device__ __forceinline__ void oriented_tile_body(const OrientKernelArgs &a, in
 #pragma unroll 1
         for (size_t j = jf; j < jend; j += CH) {
             float xs[CH], ys[CH], zs[CH];
-            if constexpr (BUF) {
+            float bs[LQ ? CH : 1];
+            if constexpr (LQ) {
+                const auto K = uniform_ptr(reinterpret_cast<const float *>(a.pack + t * a.NAp + j));
+#pragma unroll
+                for (int c = 0; c < CH; ++c) {
+                    xs[c] = K[4 * c];
+                    ys[c] = K[4 * c + 1];
+                    zs[c] = K[4 * c + 2];
+                    bs[c] = K[4 * c + 3];
+                }
+            } else if constexpr (BUF) {
                 const __amdgpu_buffer_rsrc_t rx =
                     __builtin_amdgcn_make_buffer_rsrc((void *)(X + j * a.NFp), (short)0, rows, kBufferDword3);
                 const __amdgpu_buffer_rsrc_t ry =
@@ -191,7 +220,7 @@ __device__ __forceinline__ void oriented_tile_body(const OrientKernelArgs &a, in
                 float bk[VS];
 #pragma unroll
                 for (int k = 0; k < VS; ++k)
-                    bk[k] = PER_ROW_B ? B[(size_t)min(sbase + k, a.ns - 1) * a.NAp + j + c] : B[j + c];
+                    bk[k] = PER_ROW_B ? B[(size_t)min(sbase + k, a.ns - 1) * a.NAp + j + c] : LQ ? bs[LQ ? c : 0] : B[j + c];
 #pragma unroll
                 for (int i = 0; i < VM; ++i) {
                     double d = ux[i] * xd;
@@ -320,31 +349,35 @@ __device__ __forceinline__ void oriented_tile_body(const OrientKernelArgs &a, in
                     xr = tr[i][k];
                     xi = ti[i][k];
                 }
-                a.amp[((size_t)sp * a.V + v) * a.NFp + t] = make_float2((float)xr, (float)xi);
+                if constexpr (LQ)
+                    a.parts[(((size_t)sp * a.sub + part) * a.V + v) * a.NF + t] = make_double2(xr, xi);
+                else
+                    a.amp[((size_t)sp * a.V + v) * a.NFp + t] = make_float2((float)xr, (float)xi);
             }
         }
 }
 
 // A tile of a residual-corrected call, in the mode its line asks for.
-template <int VM, int VS>
+template <int VM, int VS, bool LQ = false>
 __device__ __forceinline__ void residual_tile(const OrientKernelArgs &a, int ft, int sp, int og, int sbase,
-                                              double *__restrict__ tot) {
+                                              double *__restrict__ tot, int part = 0) {
     switch (tile_flags(a, sbase)) {
-        case 0: oriented_tile_body<VM, VS, false, 3, true>(a, ft, sp, og, sbase, tot); break;
-        case kTileCorrectUp: oriented_tile_body<VM, VS, false, 4, true>(a, ft, sp, og, sbase, tot); break;
-        case kTileCorrectDown: oriented_tile_body<VM, VS, false, 5, true>(a, ft, sp, og, sbase, tot); break;
-        default: oriented_tile_body<VM, VS, false, 2, true>(a, ft, sp, og, sbase, tot); break;
+        case 0: oriented_tile_body<VM, VS, false, 3, true, LQ>(a, ft, sp, og, sbase, tot, part); break;
+        case kTileCorrectUp: oriented_tile_body<VM, VS, false, 4, true, LQ>(a, ft, sp, og, sbase, tot, part); break;
+        case kTileCorrectDown: oriented_tile_body<VM, VS, false, 5, true, LQ>(a, ft, sp, og, sbase, tot, part); break;
+        default: oriented_tile_body<VM, VS, false, 2, true, LQ>(a, ft, sp, og, sbase, tot, part); break;
     }
 }
 
 // Modes 0 and 1 (the mode is uniform over a launch or a trajectory); modes
 // 2-5 have kernels of their own, since they need `tot` in LDS.
-template <int VM, int VS, bool PER_ROW_B, bool BUF = true>
-__device__ __forceinline__ void oriented_tile(const OrientKernelArgs &a, int ft, int sp, int og, int sbase) {
+template <int VM, int VS, bool PER_ROW_B, bool BUF = true, bool LQ = false>
+__device__ __forceinline__ void oriented_tile(const OrientKernelArgs &a, int ft, int sp, int og, int sbase,
+                                              int part = 0) {
     if (a.ap)
-        oriented_tile_body<VM, VS, PER_ROW_B, 1, BUF>(a, ft, sp, og, sbase, nullptr);
+        oriented_tile_body<VM, VS, PER_ROW_B, 1, BUF, LQ>(a, ft, sp, og, sbase, nullptr, part);
     else
-        oriented_tile_body<VM, VS, PER_ROW_B, 0, BUF>(a, ft, sp, og, sbase, nullptr);
+        oriented_tile_body<VM, VS, PER_ROW_B, 0, BUF, LQ>(a, ft, sp, og, sbase, nullptr, part);
 }
 
 }  // namespace sx

@@ -468,7 +468,12 @@ int run_batch(sx_ctx *c, int ns, size_t NM, const double *qv, const double *qlen
     if (!self) {
         const int vb = pick_vector_block(c);
         int shape = 0;
-        if (oriented && !mp) {
+        // few frames: one orientation a lane (no trials of tile shapes, which
+        // run the other form)
+        bool few = oriented && !mp && !c->noalloc && sx::few_frames(NF, c->NFp, (int)NM);
+        if (few && c->cfg.tile_shape == 0) {
+            shape = default_shape(c, ns, b_shell != nullptr);
+        } else if (oriented && !mp) {
             int rc = pick_shape(c, ns, (int)NM, bptr, b_shell != nullptr, &shape);
             if (rc != SX_OK) return rc;
         }
@@ -487,7 +492,12 @@ int run_batch(sx_ctx *c, int ns, size_t NM, const double *qv, const double *qlen
             if (rc != SX_OK) return rc;
         }
         const size_t split_stride = (size_t)V * c->NFp;
-        SX_HIP(c, c->amp.ensure(sizeof(float2) * split_stride * split));
+        int sub = 1;
+        if (few) {
+            sub = sx::few_parts(NF, c->NAp, (int)NM, ns, split, shape);
+            few = sizeof(double2) * (size_t)V * NF * split * sub <= kAmpBudgetBytes;
+        }
+        SX_HIP(c, c->amp.ensure(sizeof(float2) * split_stride * (few ? 1 : split)));
         if (mp) {
             SX_HIP(c, c->mpmom.ensure(sizeof(int) * mp->moments.size()));
             SX_HIP(c, hipMemcpyAsync(c->mpmom.p, mp->moments.data(), sizeof(int) * mp->moments.size(),
@@ -589,7 +599,14 @@ int run_batch(sx_ctx *c, int ns, size_t NM, const double *qv, const double *qlen
             int plain = 0;
             int urc = upload_tile_lines(c, ns, shape, &plain);
             if (urc != SX_OK) return urc;
-            SX_HIP(c, sx::launch_amp_oriented(oa, c->stream));
+            if (few) {
+                SX_HIP(c, c->pack.ensure(sizeof(float4) * c->NAp * NF));
+                SX_HIP(c, c->fparts.ensure(sizeof(double2) * (size_t)V * NF * split * sub));
+                SX_HIP(c, sx::launch_amp_few(oa, NF, sub, c->pack.as<float4>(), c->fparts.as<double2>(), c->stream));
+                split = 1;  // the ranges are added
+            } else {
+                SX_HIP(c, sx::launch_amp_oriented(oa, c->stream));
+            }
             c->timing.tile_shape = shape + 1;
             c->timing.shell_progression = oa.ap ? 1 : 0;
             c->timing.shell_residuals = oa.ap == 2 ? 1 : 0;
@@ -881,7 +898,7 @@ void sx_destroy(sx_ctx *c) {
     if (!c) return;
     (void)hipSetDevice(c->cfg.device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
-    for (DevBuf *d : {&c->coords, &c->b, &c->twL, &c->twL64, &c->twp, &c->twp64, &c->tw64, &c->w, &c->aidx, &c->apair, &c->tail, &c->qrev, &c->qlen, &c->uvec, &c->brow, &c->bshell, &c->mpmom, &c->mpq, &c->mpsph, &c->mpj, &c->mpjt, &c->mptab, &c->mpsum, &c->qres, &c->redbuf, &c->amp,
+    for (DevBuf *d : {&c->coords, &c->b, &c->twL, &c->twL64, &c->twp, &c->twp64, &c->tw64, &c->w, &c->aidx, &c->apair, &c->tail, &c->qrev, &c->qlen, &c->uvec, &c->brow, &c->bshell, &c->mpmom, &c->mpq, &c->mpsph, &c->mpj, &c->mpjt, &c->mptab, &c->mpsum, &c->qres, &c->redbuf, &c->pack, &c->fparts, &c->amp,
                       &c->ppart, &c->apart, &c->fqt, &c->fq, &c->fq2, &c->stage, &c->stage2})
         d->release();
     for (auto &e : c->ev)

@@ -749,80 +749,107 @@ hipError_t launch_final(const FinalArgs &a, hipStream_t stream) {
 
 // ------------------------------------------------- square / plain series ---
 
-// fqt(t) = (1/NM) sum_m S_m(t), S = |A|^2 (square, smath.cpp:168-177) or A (plain)
-__global__ __launch_bounds__(256) void series_fqt_kernel(int mode, const float2 *__restrict__ amp, size_t NFp,
-                                                         int split, size_t split_stride, int NF, int NM,
-                                                         double *__restrict__ fqt, double norm) {
-    const int s = blockIdx.y;
-    const int t = blockIdx.x * 256 + threadIdx.x;
-    if (t >= NF) return;
+// The series kernels give the lanes of a wavefront to frames and, where there
+// are fewer than 64 of these, to several vectors at once: T lanes a vector.
+__device__ __forceinline__ int series_lanes(int NF) {
+    int T = 1;
+    while (T < kWave && T < NF) T <<= 1;
+    return T;
+}
+
+// S(t) = |A|^2 (mode 1: square, smath.cpp:168-177) or A (plain) from the partial amplitudes at p
+__device__ __forceinline__ double2 series_value(int mode, const float2 *__restrict__ p, int split,
+                                                size_t split_stride) {
+    float2 x = p[0];
+    for (int k = 1; k < split; ++k) {
+        const float2 y = p[(size_t)k * split_stride];
+        x.x += y.x;
+        x.y += y.y;
+    }
+    return mode == 1 ? make_double2((double)x.x * x.x + (double)x.y * x.y, 0.0) : make_double2(x.x, x.y);
+}
+
+// fqt(t) = (1/NM) sum_m S_m(t): 64 frames (or all, if fewer) of a shell a block,
+// the vectors dealt out to its 16 wavefronts and, for few frames, to groups of
+// lanes.  One frame, 500 vectors x 10 partial amplitudes x 40 shells took 1.16 ms
+// with one thread a frame.
+constexpr int kSeriesThreads = 1024;
+__global__ __launch_bounds__(kSeriesThreads) void series_fqt_kernel(int mode, const float2 *__restrict__ amp,
+                                                                    size_t NFp, int split, size_t split_stride, int NF,
+                                                                    int NM, double *__restrict__ fqt, double norm) {
+    __shared__ double2 sh[kSeriesThreads];
+    const int s = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int T = series_lanes(NF), tl = lane & (T - 1);
+    const int t = blockIdx.x * kWave + tl;
+    double2 x = make_double2(0.0, 0.0);
+    if (t < NF)
+        for (int m = wave * (kWave / T) + lane / T; m < NM; m += (kSeriesThreads / kWave) * (kWave / T)) {
+            const double2 v = series_value(mode, amp + ((size_t)s * NM + m) * NFp + t, split, split_stride);
+            x.x += v.x;
+            x.y += v.y;
+        }
+    for (int off = T; off < kWave; off <<= 1) {
+        x.x += __shfl_xor(x.x, off, 64);
+        x.y += __shfl_xor(x.y, off, 64);
+    }
+    sh[threadIdx.x] = x;
+    __syncthreads();
+    if (threadIdx.x >= T || t >= NF) return;
     double re = 0.0, im = 0.0;
-    for (int m = 0; m < NM; ++m) {
-        const size_t v = (size_t)s * NM + m;
-        float2 x = amp[v * NFp + t];
-        for (int k = 1; k < split; ++k) {
-            const float2 y = amp[(size_t)k * split_stride + v * NFp + t];
-            x.x += y.x;
-            x.y += y.y;
-        }
-        if (mode == 1) {
-            re += (double)x.x * x.x + (double)x.y * x.y;
-        } else {
-            re += x.x;
-            im += x.y;
-        }
+    for (int w = 0; w < kSeriesThreads / kWave; ++w) {
+        re += sh[w * kWave + lane].x;
+        im += sh[w * kWave + lane].y;
     }
     fqt[((size_t)s * NF + t) * 2] = re * norm;
     fqt[((size_t)s * NF + t) * 2 + 1] = im * norm;
 }
 
-// per chunk of vectors: sum_m a_m and sum_m |a_m|^2 with a_m = mean_t S_m(t)
+// per chunk of vectors: sum_m a_m and sum_m |a_m|^2 with a_m = mean_t S_m(t),
+// T lanes a vector
 __global__ __launch_bounds__(256) void series_mean_kernel(int mode, const float2 *__restrict__ amp, size_t NFp,
                                                           int split, size_t split_stride, int NF, int NM,
                                                           int chunks, double *__restrict__ apart) {
     __shared__ double2 red[4];
     const int s = blockIdx.x / chunks, c = blockIdx.x % chunks;
     const int m0 = (int)((long)NM * c / chunks), m1 = (int)((long)NM * (c + 1) / chunks);
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int T = series_lanes(NF), tl = lane & (T - 1), group = kWave / T;
     double sa_r = 0.0, sa_i = 0.0, sa2 = 0.0;
-    for (int m = m0; m < m1; ++m) {
-        const size_t v = (size_t)s * NM + m;
+    for (int mb = m0 + (tid >> 6) * group; mb < m1; mb += 4 * group) {
+        const int m = mb + lane / T;
         double re = 0.0, im = 0.0;
-        for (int t = tid; t < NF; t += 256) {
-            float2 x = amp[v * NFp + t];
-            for (int k = 1; k < split; ++k) {
-                const float2 y = amp[(size_t)k * split_stride + v * NFp + t];
-                x.x += y.x;
-                x.y += y.y;
+        if (m < m1)
+            for (int t = tl; t < NF; t += T) {
+                const double2 v = series_value(mode, amp + ((size_t)s * NM + m) * NFp + t, split, split_stride);
+                re += v.x;
+                im += v.y;
             }
-            if (mode == 1) {
-                re += (double)x.x * x.x + (double)x.y * x.y;
-            } else {
-                re += x.x;
-                im += x.y;
-            }
+        for (int off = T >> 1; off > 0; off >>= 1) {
+            re += __shfl_xor(re, off, 64);
+            im += __shfl_xor(im, off, 64);
         }
-        const double2 r = block_sum2(re, im, red, tid, 256);
-        if (tid == 0) {
-            const double ar = r.x / NF, ai = r.y / NF;
+        if (tl == 0) {
+            const double ar = re / NF, ai = im / NF;
             sa_r += ar;
             sa_i += ai;
             sa2 += ar * ar + ai * ai;
         }
     }
+    const double2 r = block_sum2(sa_r, sa_i, red, tid, 256);
+    const double2 r2 = block_sum2(sa2, 0.0, red, tid, 256);
     if (tid == 0) {
         double *ap = apart + ((size_t)s * chunks + c) * 4;
-        ap[0] = sa_r;
-        ap[1] = sa_i;
-        ap[2] = sa2;
+        ap[0] = r.x;
+        ap[1] = r.y;
+        ap[2] = r2.x;
         ap[3] = 0.0;
     }
 }
 
 hipError_t launch_series_all(int mode, const float2 *amp, size_t NFp, int split, size_t split_stride, int NF, int NM,
                              int nshells, int chunks, double *fqt, double *apart, double norm, hipStream_t stream) {
-    hipLaunchKernelGGL(series_fqt_kernel, dim3((unsigned)((NF + 255) / 256), (unsigned)nshells), dim3(256), 0,
-                       stream, mode, amp, NFp, split, split_stride, NF, NM, fqt, norm);
+    hipLaunchKernelGGL(series_fqt_kernel, dim3((unsigned)((NF + kWave - 1) / kWave), (unsigned)nshells),
+                       dim3(kSeriesThreads), 0, stream, mode, amp, NFp, split, split_stride, NF, NM, fqt, norm);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(series_mean_kernel, dim3((unsigned)(nshells * chunks)), dim3(256), 0, stream, mode, amp,

@@ -167,6 +167,12 @@ constexpr double kTwoPiTurns = 6.283185307179586476925286766559;
 int shell_progression(const double *qlen, int ns, double rmax, ShellGrid *g);
 constexpr int kOrientShapes = 5;
 hipError_t launch_amp_oriented(const OrientArgs &a, hipStream_t stream);
+// Trajectories of few frames (few_frames): one orientation a lane.  Each atom
+// range is summed in `sub` parts (parts: [split * sub][ns * NM][NF]; pack:
+// [NF][NAp]); the ranges' amplitudes arrive added, in a.amp as of one range.
+bool few_frames(size_t NF, size_t NFp, int NM);
+int few_parts(size_t NF, size_t NAp, int NM, int ns, int split, int shape);
+hipError_t launch_amp_few(const OrientArgs &a, int NF, int sub, float4 *pack, double2 *parts, hipStream_t stream);
 int oriented_base_blocks(size_t NFp, int NM, int ns, int shape);
 // Workgroups of the oriented kernel of this shape (and stepping mode) that fit one CU at once.
 hipError_t oriented_blocks_per_cu(int shape, bool per_row, int mode, int *blocks);
