@@ -76,13 +76,12 @@ typedef struct sx_config {
     int multipole_terms; /* multipole: the spherical (sphere, 36 B) or cylinder-frame
                             (cylinder, 12 B) coordinates of every (atom, frame) 1 formed once
                             per call in a pre-pass, 2 formed by the amplitude kernel itself;
-                            0 picks 1 up to 16 GB of terms, else 2.  With 0 and 1 the Bessel
-                            functions of every (shell, atom, frame) are formed once per call:
-                            sphere, degrees up to 16, inside a kernel that sums products of
-                            radial and angular factors; cylinder, orders up to 32, in a
-                            pre-pass (8 B each) while that table stays within 96 GB and leaves
-                            4 GB of device memory free; 3 is 1 without these (the two lowest
-                            only, the rest by recurrence in the kernel) */
+                            0 picks 1 up to 16 GB of terms, else 2.  With 0 and 1, sphere lists
+                            of degrees up to 16 and cylinder lists of Bessel orders up to 32 run
+                            as sums of products whose factors are formed once per (atom, frame,
+                            shell), while their FP64 partial sums stay within 96 GB and leave
+                            4 GB of device memory free; 3 is 1 without these (every wavefront of
+                            8 moments runs its own recurrences) */
     int reserved[6];
 } sx_config;
 

@@ -130,11 +130,10 @@ int pick_split(const sx_ctx *c, int V, int vb) {
 constexpr size_t kSplitAmpBudget = (size_t)4 << 30;
 // Largest buffer of per-(atom, frame) spherical terms of the sphere multipole path.
 constexpr size_t kSphereTermBudget = (size_t)16 << 30;
-// The cylinder's table of J_n per (shell, order, atom, frame) and the sphere's
-// partial sums: at most this much, and only while this much device memory
-// stays free beside it.
-constexpr size_t kBesselTableBudget = (size_t)96 << 30;
-constexpr size_t kBesselTableMargin = (size_t)4 << 30;
+// The partial sums of a multipole call: at most this much, and only while
+// this much device memory stays free beside them.
+constexpr size_t kMultipoleSumBudget = (size_t)96 << 30;
+constexpr size_t kMultipoleSumMargin = (size_t)4 << 30;
 
 // Splits from `first` to 16 (at least 64 atoms a range, partial amplitude
 // sets of split_bytes each within kSplitAmpBudget) for `base` equal
@@ -157,13 +156,13 @@ int round_filling_split(long base, int first, long resident, size_t NAp, size_t 
 }
 
 // Whether `buf` may hold `bytes`: within the budget, and with
-// kBesselTableMargin of device memory left beside it.
+// kMultipoleSumMargin of device memory left beside it.
 bool multipole_buffer_fits(const DevBuf &buf, size_t bytes) {
-    if (bytes > kBesselTableBudget) return false;
+    if (bytes > kMultipoleSumBudget) return false;
     if (buf.p && bytes <= buf.cap) return true;
     size_t fr = 0, tot = 0;
     if (hipMemGetInfo(&fr, &tot) != hipSuccess) return false;
-    return fr + buf.cap >= bytes + kBesselTableMargin;
+    return fr + buf.cap >= bytes + kMultipoleSumMargin;
 }
 
 // Atom ranges of a multipole call, each of which rounds its amplitudes to
@@ -541,51 +540,56 @@ int run_batch(sx_ctx *c, int ns, size_t NM, const double *qv, const double *qlen
                 else
                     SX_HIP(c, sx::launch_multipole_cylinder_terms(ma, c->mpsph.p, c->stream));
                 ma.sph = c->mpsph.p;
-                // sphere, degrees up to 16: sums of products of radial and
-                // angular factors
-                sx::SpherePlan sp;
-                int sub = 0;
-                if (mp->kind == 0 && terms != 3 && sx::sphere_sums_grid_fits(ns, split) &&
-                    *std::max_element(mp->qinfo.begin(), mp->qinfo.end()) * c->rmax < 0.99 * sx::kSphereMaxArg &&
-                    sx::make_sphere_plan(mp->moments.data(), (int)NM, ns, &sp)) {
-                    int cus = 0;
-                    SX_HIP(c, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->cfg.device));
-                    sub = sx::sphere_parts_per_range(sp, c->NFp, c->NAp, split, std::max(cus, 1));
-                    while (sub > 0 &&
-                           !multipole_buffer_fits(c->mpsum, sx::sphere_parts_bytes(sp, c->NFp, ns, split, sub)))
-                        sub /= 2;
-                }
-                // cylinder up to order 32: every Bessel function of every
-                // (shell, atom, frame) once per call when the table fits; else
-                // (and for the sphere above degree 16) the two lowest (16 B
-                // each) within the terms' budget
+                // degrees up to 16 (sphere) or orders up to 32 (cylinder): sums of
+                // products, each range in `sub` FP64 parts; else, and where the
+                // parts find no room, the moments' own recurrences
                 int N1 = 1;
+                double qmax = 0.0;
                 if (mp->kind == 1) {
                     for (size_t k = 0; k + 1 < mp->moments.size(); k += 2) {
                         const int l = mp->moments[k], m = mp->moments[k + 1];
                         const int n = (l == 0 || m > 3 || m < 0) ? 0 : (m <= 1 ? 2 * l : 2 * l - 1);
                         N1 = std::max(N1, n + 1);
                     }
+                    for (int s = 0; s < ns; ++s)
+                        qmax = std::max({qmax, mp->qinfo[3 * s], std::fabs(mp->qinfo[3 * s + 2])});
+                } else {
+                    qmax = *std::max_element(mp->qinfo.begin(), mp->qinfo.end());
                 }
-                // (the table also holds two phases per (shell, atom, frame))
-                const size_t tab_bytes =
-                    (sizeof(double) * (size_t)N1 + 2 * sizeof(double2)) * (size_t)ns * c->NAp * c->NFp;
+                int cus = 0;
+                SX_HIP(c, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->cfg.device));
+                cus = std::max(cus, 1);
+                sx::SpherePlan sp;
+                int sub = 0;
+                if (terms != 3 && qmax * c->rmax < 0.99 * sx::kMultipoleMaxArg) {
+                    if (mp->kind == 0 && sx::sphere_sums_grid_fits(ns, split) &&
+                        sx::make_sphere_plan(mp->moments.data(), (int)NM, ns, &sp))
+                        sub = sx::sphere_parts_per_range(sp, c->NFp, c->NAp, split, cus);
+                    else if (mp->kind == 1 && N1 <= sx::kCylinderSumN1 && sx::cylinder_sums_grid_fits((int)NM, ns, split))
+                        sub = sx::cylinder_parts_per_range(N1, c->NFp, c->NAp, ns, split, cus);
+                }
+                auto part_bytes = [&](int parts) {
+                    return mp->kind == 0 ? sx::sphere_parts_bytes(sp, c->NFp, ns, split, parts)
+                                         : sx::cylinder_parts_bytes(N1, c->NFp, ns, split, parts);
+                };
+                while (sub > 0 && !multipole_buffer_fits(c->mpsum, part_bytes(sub))) sub /= 2;
+                const size_t angle_bytes = mp->kind == 1 ? sizeof(double2) * c->NAp * c->NFp : 0;
+                if (sub > 0 && angle_bytes > 0 && !multipole_buffer_fits(c->mpang, angle_bytes + part_bytes(sub))) sub = 0;
                 const size_t j01_bytes = sizeof(double2) * (size_t)ns * c->NAp * c->NFp;
                 if (sub > 0) {
-                    std::vector<char> tables(sx::sphere_table_bytes(sp));
-                    sx::sphere_tables(sp, tables.data());
-                    SX_HIP(c, c->mptab.ensure(tables.size()));
-                    SX_HIP(c, hipMemcpyAsync(c->mptab.p, tables.data(), tables.size(), hipMemcpyHostToDevice,
-                                             c->stream));
-                    SX_HIP(c, c->mpsum.ensure(sx::sphere_parts_bytes(sp, c->NFp, ns, split, sub)));
-                    SX_HIP(c, sx::launch_sphere_sums(ma, sp, c->mptab.p, sub, c->mpsum.p, c->stream));
+                    SX_HIP(c, c->mpsum.ensure(part_bytes(sub)));
+                    if (mp->kind == 0) {
+                        std::vector<char> tables(sx::sphere_table_bytes(sp));
+                        sx::sphere_tables(sp, tables.data());
+                        SX_HIP(c, c->mptab.ensure(tables.size()));
+                        SX_HIP(c, hipMemcpyAsync(c->mptab.p, tables.data(), tables.size(), hipMemcpyHostToDevice,
+                                                 c->stream));
+                        SX_HIP(c, sx::launch_sphere_sums(ma, sp, c->mptab.p, sub, c->mpsum.p, c->stream));
+                    } else {
+                        SX_HIP(c, c->mpang.ensure(angle_bytes));
+                        SX_HIP(c, sx::launch_cylinder_sums(ma, N1, sub, c->mpang.p, c->mpsum.p, c->stream));
+                    }
                     summed = true;
-                } else if (mp->kind == 1 && terms != 3 && N1 <= sx::kCylTableN1 &&
-                           multipole_buffer_fits(c->mpjt, tab_bytes)) {
-                    SX_HIP(c, c->mpjt.ensure(tab_bytes));
-                    SX_HIP(c, sx::launch_multipole_bessel_table(ma, N1, c->mpjt.p, c->stream));
-                    ma.jtab = c->mpjt.p;
-                    ma.jl1 = N1;
                 } else if (j01_bytes <= kSphereTermBudget) {
                     SX_HIP(c, c->mpj.ensure(j01_bytes));
                     SX_HIP(c, sx::launch_multipole_bessel01(ma, c->mpj.p, c->stream));
@@ -898,7 +902,7 @@ void sx_destroy(sx_ctx *c) {
     if (!c) return;
     (void)hipSetDevice(c->cfg.device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
-    for (DevBuf *d : {&c->coords, &c->b, &c->twL, &c->twL64, &c->twp, &c->twp64, &c->tw64, &c->w, &c->aidx, &c->apair, &c->tail, &c->qrev, &c->qlen, &c->uvec, &c->brow, &c->bshell, &c->mpmom, &c->mpq, &c->mpsph, &c->mpj, &c->mpjt, &c->mptab, &c->mpsum, &c->qres, &c->redbuf, &c->pack, &c->fparts, &c->amp,
+    for (DevBuf *d : {&c->coords, &c->b, &c->twL, &c->twL64, &c->twp, &c->twp64, &c->tw64, &c->w, &c->aidx, &c->apair, &c->tail, &c->qrev, &c->qlen, &c->uvec, &c->brow, &c->bshell, &c->mpmom, &c->mpq, &c->mpsph, &c->mpj, &c->mpang, &c->mptab, &c->mpsum, &c->qres, &c->redbuf, &c->pack, &c->fparts, &c->amp,
                       &c->ppart, &c->apart, &c->fqt, &c->fq, &c->fq2, &c->stage, &c->stage2})
         d->release();
     for (auto &e : c->ev)

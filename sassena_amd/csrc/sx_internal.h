@@ -289,19 +289,28 @@ struct MultipoleArgs {
     // (cylinder) per (shell, atom, frame) from launch_multipole_bessel01, or
     // nullptr to form them in the kernel
     const void *cj01 = nullptr;
-    // cylinder: J_n for n < jl1 per (shell, order, atom, frame) from
-    // launch_multipole_bessel_table, or nullptr
-    const void *jtab = nullptr;
-    int jl1 = 0;
 };
+// Largest argument of the Bessel functions and phases of the multipole sums.
+constexpr double kMultipoleMaxArg = 1e5;
+
+// The cylinder average as sums per Bessel order, for orders below
+// kCylinderSumN1 and arguments up to kMultipoleMaxArg, from the cylinder terms
+// (m.sph) and [NAp][NFp] double2 of work memory for the angles; parts of the
+// ranges as for the sphere below.
+constexpr int kCylinderSumN1 = 33;
+inline bool cylinder_sums_grid_fits(int nmo, int ns, int split) { return nmo <= 65535 && (size_t)ns * split <= 65535; }
+int cylinder_parts_per_range(int N1, size_t NFp, size_t NAp, int ns, int split, int cus);
+size_t cylinder_parts_bytes(int N1, size_t NFp, int ns, int split, int sub);
+hipError_t launch_cylinder_sums(const MultipoleArgs &m, int N1, int sub, void *angles, void *parts,
+                                hipStream_t stream);
+
 // The sphere average as sums of products of radial and angular factors, for
 // moment lists of degrees below kSphereSumL1 and arguments |q| r up to
-// kSphereMaxArg: its schedule and tables (host), and the launch, from the
+// kMultipoleMaxArg: its schedule and tables (host), and the launch, from the
 // sphere terms (m.sph).  Each atom range is summed in `sub` parts in FP64
 // (parts, sphere_parts_bytes), which are added before the amplitude of the
 // range is rounded to FP32.
 constexpr int kSphereSumL1 = 17;
-constexpr double kSphereMaxArg = 1e5;
 // What a wavefront does for one degree l of two orders m, m + 1 (m even).
 struct SphereEntry {
     double alpha1, alpha2;  // recurrence coefficients of the two orders at l
@@ -330,14 +339,6 @@ hipError_t launch_sphere_sums(const MultipoleArgs &m, const SpherePlan &p, const
                               hipStream_t stream);
 
 hipError_t launch_multipole(const MultipoleArgs &m, hipStream_t stream);
-// Orders the cylinder's Bessel table holds at most (n <= 32, the orders 2l
-// and 2l - 1 of l <= 16).
-constexpr int kCylTableN1 = 33;
-// J_0 .. J_{L1-1} of every (shell, atom, frame) of a cylinder call from its
-// terms (m.sph), into out[(s L1 + n) NAp NFp + atom NFp + frame] (FP64), then
-// (cos, sin) of sgn z q_z and of phi - q_phi per (shell, 2, atom, frame) as
-// double2 (32 B per (shell, atom, frame) more).
-hipError_t launch_multipole_bessel_table(const MultipoleArgs &m, int L1, void *out, hipStream_t stream);
 // Workgroups of the multipole kernel that fit one CU, and its workgroups per
 // atom range (kind 0, sphere: kSphereShells shells per workgroup).
 constexpr int kSphereShells = 2;

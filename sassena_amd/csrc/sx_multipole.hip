@@ -43,9 +43,6 @@ struct MultipoleKernelArgs {
     const double *sct, *sst, *ssp, *scp;  // cos theta, sin theta, sin phi, cos phi
     const float *cphi, *cz;  // cylinder terms (r in srf), float-rounded as the reference stages them
     const double2 *cj01;     // j_0, j_1 (sphere) or J_0, J_1 (cylinder) per (shell, atom, frame), or nullptr
-    const double *jtab;      // cylinder: J_n per (shell, order, atom, frame), or nullptr
-    int jl1;
-    const double2 *etab;     // cylinder with jtab: (cos, sin) of sgn z q_z and of psi per (shell, 2, atom, frame)
 };
 
 // j_l(x) for the moment degrees ls[0..kMoments) of a wavefront in one
@@ -370,98 +367,6 @@ __global__ __launch_bounds__(256) void cylinder_bessel01_kernel(const float *__r
     }
 }
 
-// J_0 .. J_nhi (nhi < NT) of x >= 0 in one recurrence, as
-// cyl_bessel_orders forms each order: J_0 and J_1 as given, upward where
-// x > nhi, else Miller's recurrence from an even start above nhi normalised
-// by J_0 + 2 sum_k J_2k = 1.  Loops over the table's fixed order count with
-// guards on nhi keep every index a constant.
-template <int NT>
-__device__ __forceinline__ void cyl_bessel_all(int nhi, double x, double J0, double J1, double (&jv)[NT]) {
-#pragma unroll
-    for (int q = 0; q < NT; ++q) jv[q] = 0.0;
-    jv[0] = J0;
-    jv[1] = J1;
-    if (nhi < 2 || !(x > 1e-20)) return;
-    const double ix = 1.0 / x;
-    if (x > (double)nhi) {
-        double a = J0, bb = J1;  // J_{k-1}, J_k
-#pragma unroll
-        for (int k = 1; k + 1 < NT; ++k)
-            if (k < nhi) {
-                const double nx = (2.0 * k) * ix * bb - a;
-                a = bb;
-                bb = nx;
-                jv[k + 1] = bb;
-            }
-        return;
-    }
-    int N = nhi + 32 + (int)(2.0 * sqrt(2.0 * (double)nhi));
-    N += N & 1;  // even: the normalisation sums even orders
-    double fp1 = 0.0, f = 1e-280, norm = 0.0;
-    // f <- J_{k-1} (unnormalised), 2 J_{k-1} into the sum when k - 1 is even and positive
-    auto step = [&](int k) {
-        const double fm1 = (2.0 * k) * ix * f - fp1;
-        fp1 = f;
-        f = fm1;
-        if (((k - 1) & 1) == 0 && k > 1) norm += 2.0 * f;
-        if (fabs(f) > 1e250) {
-            f *= 1e-250;
-            fp1 *= 1e-250;
-            norm *= 1e-250;
-#pragma unroll
-            for (int q = 0; q < NT; ++q) jv[q] *= 1e-250;
-        }
-    };
-    int k = N;
-    for (; k > nhi + 1; --k) step(k);
-    // k = nhi + 1: each step now yields an order to keep
-#pragma unroll
-    for (int o = NT - 1; o >= 0; --o)
-        if (o <= nhi) {
-            step(o + 1);  // f = J_o
-            jv[o] = f;
-        }
-    norm += f;  // J_0
-    const double inorm = 1.0 / norm;
-#pragma unroll
-    for (int q = 2; q < NT; ++q)
-        if (q <= nhi) jv[q] *= inorm;
-    jv[0] = J0;
-    jv[1] = J1;
-}
-
-// J_0 .. J_{N1-1} of q_r r for every (shell, atom, frame) of a cylinder call
-// (out[(s N1 + n) NAp NFp + e]), from the cylinder terms (r rounded to float):
-// formed once per call instead of once per moment block.
-// NT: orders the thread holds (at least N1; 21 covers the moments up to l = 10).
-// Also the two phases of every (shell, atom, frame), by the amplitude
-// kernel's own expressions: ex[(2 s) n + e] = (cos, sin)(sgn z q_z),
-// ex[(2 s + 1) n + e] = (cos, sin)(phi - q_phi).
-template <int NT>
-__global__ __launch_bounds__(256, NT <= 21 ? 3 : 2) void cylinder_bessel_table_kernel(
-    const float *__restrict__ rr, const float *__restrict__ cphi, const float *__restrict__ cz, size_t n,
-    const double *__restrict__ qinfo, int ns, int N1, double *__restrict__ out, double2 *__restrict__ ex) {
-    const size_t e = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (e >= n) return;
-    const double rf = rr[e], phif = cphi[e], zf = cz[e];
-    for (int s = 0; s < ns; ++s) {
-        const double qphi = qinfo[3 * s + 1], qz = qinfo[3 * s + 2];
-        double sgn = 1.0;
-        if ((zf != 0) && (qz != 0)) sgn = (zf * qz) / (fabs(zf) * fabs(qz));
-        double exs, exc, sp1, cp1;
-        sincos(sgn * zf * qz, &exs, &exc);
-        sincos(phif - qphi, &sp1, &cp1);
-        ex[(size_t)(2 * s) * n + e] = make_double2(exc, exs);
-        ex[(size_t)(2 * s + 1) * n + e] = make_double2(cp1, sp1);
-        const double p = rf * qinfo[3 * s];
-        double jv[NT];
-        cyl_bessel_all<NT>(N1 - 1, p, j0(p), j1(p), jv);
-#pragma unroll
-        for (int q = 0; q < NT; ++q)
-            if (q < N1) out[((size_t)s * N1 + q) * n + e] = jv[q];
-    }
-}
-
 // KIND 0 sphere, 1 cylinder, each instantiated on its own.  Both are bound by
 // the latency of serial FP64 recurrences, so they are held to 3 (sphere) and
 // 2 (cylinder) wavefronts per SIMD, the bounds that measured fastest despite
@@ -659,51 +564,23 @@ __global__ __launch_bounds__(256, KIND == 0 ? 3 : 2) void multipole_kernel(Multi
                 phif = (float)phi;
                 zf = (float)zz;
             }
-            const size_t plane = a.NAp * a.NFp, e = j * a.NFp + t;
-            double exs, exc;
-            if constexpr (SRC == 3) {
-                const double2 ee = a.etab[(size_t)(2 * s) * plane + e];
-                exc = ee.x;
-                exs = ee.y;
-            } else {
-                double sgn = 1.0;
-                if ((zf != 0) && (qz != 0)) sgn = (zf * qz) / (fabs(zf) * fabs(qz));
-                sincos(sgn * zf * qz, &exs, &exc);
-            }
+            double exs, exc, sgn = 1.0;
+            if ((zf != 0) && (qz != 0)) sgn = (zf * qz) / (fabs(zf) * fabs(qz));
+            sincos(sgn * zf * qz, &exs, &exc);
             const double p = rf * qr, psi = phif - qphi;
             double jn[kMoments];
-            if constexpr (SRC == 3) {
-                // the moments' orders from the table, one load per distinct order
-                double cur = 0.0;
-                int np = -1;
-#pragma unroll
-                for (int k = 0; k < kMoments; ++k) {
-                    if (cn[k] != np) {
-                        np = cn[k];
-                        cur = a.jtab[((size_t)s * a.jl1 + np) * plane + e];
-                    }
-                    jn[k] = cur;
-                }
+            double J0, J1;
+            if constexpr (SRC == 2) {
+                const double2 jj = a.cj01[((size_t)s * a.NAp + j) * a.NFp + t];
+                J0 = jj.x;
+                J1 = jj.y;
             } else {
-                double J0, J1;
-                if constexpr (SRC == 2) {
-                    const double2 jj = a.cj01[((size_t)s * a.NAp + j) * a.NFp + t];
-                    J0 = jj.x;
-                    J1 = jj.y;
-                } else {
-                    J0 = j0(p);
-                    J1 = j1(p);
-                }
-                cyl_bessel_orders(cn, nhi, p, J0, J1, jn);
+                J0 = j0(p);
+                J1 = j1(p);
             }
+            cyl_bessel_orders(cn, nhi, p, J0, J1, jn);
             double sn = 0.0, cs = 1.0, sp1, cp1;
-            if constexpr (SRC == 3) {
-                const double2 pp = a.etab[(size_t)(2 * s + 1) * plane + e];
-                cp1 = pp.x;
-                sp1 = pp.y;
-            } else {
-                sincos(psi, &sp1, &cp1);  // e^{i psi}
-            }
+            sincos(psi, &sp1, &cp1);  // e^{i psi}
 #pragma unroll
             for (int k = 0; k < kMoments; ++k) {
                 if (k >= nk) break;
@@ -785,10 +662,6 @@ hipError_t launch_multipole(const MultipoleArgs &m, hipStream_t stream) {
     k.sct = k.sst = k.ssp = k.scp = nullptr;
     k.cphi = k.cz = nullptr;
     k.cj01 = static_cast<const double2 *>(m.cj01);
-    k.jtab = static_cast<const double *>(m.jtab);
-    k.jl1 = m.jl1;
-    k.etab = m.kind == 1 && m.jtab ? reinterpret_cast<const double2 *>(k.jtab + (size_t)m.ns * m.jl1 * m.NAp * m.NFp)
-                                   : nullptr;
     if (m.sph && m.kind == 0) {
         k.srf = static_cast<const float *>(m.sph);
         const double *d = reinterpret_cast<const double *>(static_cast<const char *>(m.sph) + sizeof(float) * n);
@@ -810,8 +683,6 @@ hipError_t launch_multipole(const MultipoleArgs &m, hipStream_t stream) {
         hipLaunchKernelGGL((multipole_kernel<0, 1>), grid, dim3(256), 0, stream, k);
     else if (m.kind == 0)
         hipLaunchKernelGGL((multipole_kernel<0, 0>), grid, dim3(256), 0, stream, k);
-    else if (k.srf && k.jtab)
-        hipLaunchKernelGGL((multipole_kernel<1, 3>), grid, dim3(256), 0, stream, k);
     else if (k.srf && k.cj01)
         hipLaunchKernelGGL((multipole_kernel<1, 2>), grid, dim3(256), 0, stream, k);
     else if (k.srf)
@@ -848,22 +719,6 @@ hipError_t launch_multipole_cylinder_terms(const MultipoleArgs &m, void *terms, 
     const float *X = m.coords, *Y = m.coords + n, *Z = m.coords + 2 * n;
     hipLaunchKernelGGL(cylinder_terms_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, X, Y, Z, n,
                        m.base, rr, rr + n, rr + 2 * n);
-    return hipGetLastError();
-}
-
-hipError_t launch_multipole_bessel_table(const MultipoleArgs &m, int L1, void *out, hipStream_t stream) {
-    if (m.kind != 1 || L1 < 1 || L1 > kCylTableN1) return hipErrorInvalidValue;
-    const size_t n = m.NAp * m.NFp;
-    // the phases follow the orders: [ns][2][n] double2
-    const float *rr = static_cast<const float *>(m.sph);
-    double *J = static_cast<double *>(out);
-    double2 *ex = reinterpret_cast<double2 *>(J + (size_t)m.ns * L1 * n);
-    if (L1 <= 21)
-        hipLaunchKernelGGL(cylinder_bessel_table_kernel<21>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream,
-                           rr, rr + n, rr + 2 * n, n, m.qinfo, m.ns, L1, J, ex);
-    else
-        hipLaunchKernelGGL(cylinder_bessel_table_kernel<kCylTableN1>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
-                           stream, rr, rr + n, rr + 2 * n, n, m.qinfo, m.ns, L1, J, ex);
     return hipGetLastError();
 }
 

@@ -29,7 +29,7 @@
 #include <algorithm>
 #include <cmath>
 
-#include "sx_internal.h"
+#include "sx_special_device.h"
 
 namespace sx {
 
@@ -38,47 +38,6 @@ namespace {
 constexpr int kWaves = 8;
 constexpr int kThreads = kWaves * kWave;
 constexpr double kPi = 3.14159265358979323846;
-
-// Taylor coefficients of sin (x^17 .. x^3) and cos (x^16 .. x^4), read by scalar
-// loads: as literals they would be kept in vector registers, which the sums need.
-__constant__ const double kTaylor[15] = {
-    1.0 / 355687428096000.0, -1.0 / 1307674368000.0, 1.0 / 6227020800.0, -1.0 / 39916800.0, 1.0 / 362880.0,
-    -1.0 / 5040.0,           1.0 / 120.0,            -1.0 / 6.0,         //
-    1.0 / 20922789888000.0,  -1.0 / 87178291200.0,   1.0 / 479001600.0,  -1.0 / 3628800.0,   1.0 / 40320.0,
-    -1.0 / 720.0,            1.0 / 24.0};
-
-// Wave-uniform, read-only tables, read by scalar loads.
-template <typename T>
-__device__ __forceinline__ const __attribute__((address_space(4))) T *uniform(const T *p) {
-    return (const __attribute__((address_space(4))) T *)p;
-}
-
-// sin and cos of 0 <= x <= kSphereMaxArg: two-term reduction by pi/2 with
-// fused products (the second constant takes pi/2 to 2^-106), then the Taylor
-// series on [-pi/4, pi/4], truncated below 1e-17.
-__device__ __forceinline__ void sincos_reduced(double x, double &s, double &c) {
-    int zo = 0;
-    asm volatile("" : "+s"(zo));
-    const auto C = uniform(kTaylor) + zo;
-    const double k = rint(x * 0.63661977236758134308);
-    double r = fma(-k, 1.57079632679489661923, x);
-    r = fma(-k, 6.12323399573676603587e-17, r);
-    const double z = r * r;
-    double ps = C[0];
-#pragma unroll
-    for (int i = 1; i < 8; ++i) ps = fma(ps, z, C[i]);
-    const double sr = fma(ps * z, r, r);
-    double pc = C[8];
-#pragma unroll
-    for (int i = 9; i < 15; ++i) pc = fma(pc, z, C[i]);
-    const double cr = fma(pc * z, z, fma(-0.5, z, 1.0));
-    const int q = (int)k;
-    const bool swap = q & 1;
-    s = swap ? cr : sr;
-    c = swap ? sr : cr;
-    if (q & 2) s = -s;
-    if ((q + 1) & 2) c = -c;
-}
 
 // w j_l(x), l < L1, to J[l * stride]: upward where x exceeds the largest
 // degree, else by Miller's downward recurrence, normalised to j_0 or j_1; below 1e-8
@@ -97,10 +56,7 @@ __device__ __forceinline__ void bessel_to_lds(double w, double x, int L1, int st
     }
     double s, c;
     sincos_reduced(x, s, c);
-    // 1 / x from the hardware reciprocal by two Newton steps
-    double ix = __builtin_amdgcn_rcp(x);
-    ix = fma(fma(-x, ix, 1.0), ix, ix);
-    ix = fma(fma(-x, ix, 1.0), ix, ix);
+    const double ix = reciprocal(x);
     const double j0 = w * s * ix, j1 = fma(-w, c, j0) * ix;
     const int L = L1 - 1;
     if (x > (double)L) {

@@ -57,3 +57,34 @@ def test_sphere_sums_of_partial_lists(moments):
     moments = [mo for mo in moments if abs(mo[1]) <= mo[0]]
     bs = np.random.default_rng(1).uniform(-2, 4, size=(3, 77))
     check(*both("sphere", xyz, b, qv, moments, 1, b_shell=bs))
+
+
+@pytest.mark.parametrize("lmax,ns,NA,NF,split,axis", [
+    (0, 1, 1, 1, 1, (0, 0, 1)), (1, 3, 5, 63, 1, (0, 0, 1)), (2, 2, 33, 64, 1, (0.3, -0.2, 0.9)), (3, 5, 64, 65, 2, (0, 1, 0)),
+    (4, 4, 70, 100, 1, (0, 0, 1)), (6, 7, 200, 70, 3, (1, 2, -1)), (8, 3, 130, 30, 1, (0, 0, 1)), (10, 5, 300, 40, 2, (0, 0, -1)),
+    (12, 4, 90, 64, 1, (0, 0, 1)), (13, 2, 129, 129, 1, (0.1, 0.1, 0.5)), (16, 6, 65, 64, 1, (0, 0, 1))])
+def test_cylinder_sums(lmax, ns, NA, NF, split, axis):
+    """q_r r from 0 through the leading terms, Miller's recurrence and the
+    asymptotic start, shells along the axis and across it."""
+    xyz, b = walk(NA, NF, 100 + lmax + ns)
+    b[0] = 6.65
+    xyz[:, 0, 0] = 0.0   # r = 0
+    if NA > 3:
+        b[1:4] = 5.8
+        xyz[:, 1] *= 1e-7
+        xyz[:, 2] *= 8.0
+        xyz[:2, 3] = 0.0
+    a = np.asarray(axis, float) / np.linalg.norm(axis)
+    q = np.linspace(0.05, 3.0, ns)
+    qv = q[:, None] * np.array([0.5, -0.2, 0.8])
+    qv[0] = 1.1 * a
+    moments = [(0, 0)] + [(l, m) for l in range(1, lmax + 1) for m in range(4)]
+    check(*both("cylinder", xyz, b, qv, moments, split, axis=axis))
+
+
+def test_cylinder_sums_of_partial_lists():
+    """A list with gaps and repeats in any order, per-shell factors."""
+    xyz, b = walk(77, 90, 5)
+    qv = np.array([[0.2, 0.3, 0.0], [1.0, -0.4, 0.8], [4.0, 0.0, 0.1]])
+    bs = np.random.default_rng(1).uniform(-2, 4, size=(3, 77))
+    check(*both("cylinder", xyz, b, qv, [(7, 2), (1, 1), (0, 0), (7, 2), (11, 3), (4, 0)], 1, b_shell=bs))
