@@ -4,15 +4,24 @@
 // y = W3 . tanh(W2 tanh(W1 x + b1) + b2) + b3 with 16 inputs (zero padded),
 // two hidden layers of 128 and one output.  W1 and W2 are BF16 operands of
 // v_mfma_f32_16x16x16_bf16 (FP32 accumulation); the output layer, biases,
-// activations and optimizer state are FP32.  One wavefront owns 16 rows:
-//   forward   x[16x16] W1 -> h1[16x128]; h1 W2 -> h2[16x128]; h2 . W3 -> y
-//   backward  dW2 = h1^T dz2 and dW1 = x^T dz1 (MFMA, K = the 16 rows),
-//             dh1 = dz2 W2^T (MFMA), reductions over rows in LDS.
+// activations and optimizer state are FP32.
 // Operand layouts of the 16x16x16 MFMA (lane l, register j < 4):
 //   A[m][k]: m = l % 16, k = 4 (l / 16) + j;  B[k][n]: k = 4 (l / 16) + j,
 //   n = l % 16;  D[m][n]: m = 4 (l / 16) + j, n = l % 16.
-// A wavefront's D tile of h1 is therefore the A operand of h1^T and the B
-// operand of dz2 is its D tile, so the weight gradients need no shuffles.
+// A D tile of h1 is therefore the A operand of h1^T and a D tile of dz2 the B
+// operand of dz2, so the weight gradients need no shuffles.
+//
+// A step is bound by latency, not by its 0.5 GFLOP: a workgroup takes 64 rows
+// with 16 wavefronts, wavefront = (16 rows) x (2 of 8 column tiles), so that
+// every stage is a few MFMAs deep; the weights are kept as ready operand
+// fragments (8 B a lane, loaded at the start straight into registers);
+// activations and their derivatives pass between wavefronts through LDS, as
+// fragments for the weight gradients and as rows for the next layer; the weight
+// gradients sum their 64 rows in the accumulators and leave as fragments.  A
+// second launch sums the workgroups' partials in a fixed order and applies Adam.
+// 4,096 rows a step: 14 + 5 us (133 + 16 us when each of four wavefronts took 16
+// rows through all columns, copied W2 into LDS and added its gradients there
+// by LDS atomics).
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -29,7 +38,15 @@ namespace sxm {
 constexpr int IN = 16, H = 128;
 constexpr int OFF_W1 = 0, OFF_B1 = OFF_W1 + IN * H, OFF_W2 = OFF_B1 + H, OFF_B2 = OFF_W2 + H * H,
               OFF_W3 = OFF_B2 + H, OFF_B3 = OFF_W3 + H, NPARAM = OFF_B3 + 1;
-constexpr int ROWS_PER_BLOCK = 64;  // 4 wavefronts x 16 rows
+constexpr int ROWS_PER_BLOCK = 64;
+constexpr int kStepThreads = 1024;
+// A workgroup's gradients and loss: the 64 tiles of W2 and the 8 of W1 as
+// fragments [tile][lane][4], then b1, b2, W3, b3 and the loss, padded to 16 B.
+constexpr int PK_W2 = 0, PK_W1 = PK_W2 + H * H, PK_B1 = PK_W1 + IN * H, PK_B3 = PK_B1 + 3 * H, PK_LOSS = PK_B3 + 1,
+              PK = (PK_LOSS + 1 + 3) / 4 * 4;
+// BF16 operand fragments: W1 [nt][lane][4], W2 [nt][kt][lane][4] (B operand of
+// h1 W2), W2^T [nt][kt][lane][4] (B operand of dz2 W2^T).
+constexpr int FR_W1 = 0, FR_W2 = FR_W1 + IN * H, FR_W2T = FR_W2 + H * H, FR = FR_W2T + H * H;
 
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -64,212 +81,299 @@ struct StepArgs {
     int sample;            // 1: draw rows with pick_row, 0: rows 0..rows-1
     unsigned long long seed;
     unsigned step;
-    const short *w1b;      // BF16 copies [IN][H], [H][H]
-    const short *w2b;
+    const short *frag;     // BF16 operand fragments of W1, W2, W2^T
     const float *p;        // FP32 parameters (b1, b2, W3, b3 used from here)
     float *y;              // [rows] outputs (optional)
-    float *partial;        // [blocks][NPARAM + 1] gradient partials and loss (training)
+    float *partial;        // [blocks][PK] gradients and loss of each workgroup (training)
 };
 
+// Row stride of the row-major LDS tiles: 132 shorts, so that the 16 rows of an
+// A operand start in different banks.
+constexpr int LD = H + 4;
+
+// Sum over the four lane groups (rows of a D tile) of a per-lane column value.
+__device__ __forceinline__ float col_sum(float x) {
+    x += __shfl_xor(x, 16, 64);
+    x += __shfl_xor(x, 32, 64);
+    return x;
+}
+
 // Forward (and backward when a.t != nullptr) of ROWS_PER_BLOCK rows.
-__global__ __launch_bounds__(256) void mlp_step_kernel(StepArgs a) {
-    __shared__ short w2s[H * H];            // 32 KB, W2 as BF16 [k][n]
-    __shared__ short w1s[IN * H];           // W1 as BF16 [k][n]
-    __shared__ float gW2[H * H];            // 64 KB block accumulator of dW2
-    __shared__ float gW1[IN * H];
-    __shared__ float gsmall[3 * H + 2];     // db1, db2, dW3, db3, loss
-    __shared__ short scratch[4][16 * H];    // per-wave re-layout tile (BF16)
+__global__ __launch_bounds__(kStepThreads) void mlp_step_kernel(StepArgs a) {
+    __shared__ short rows_lds[ROWS_PER_BLOCK * LD];  // h1, then dz2: A operands
+    __shared__ bf16x4 h1f[4 * 8 * 64];               // D tiles [row tile][column tile][lane]
+    __shared__ bf16x4 dzf[4 * 8 * 64];               // dz2, then dz1
+    __shared__ bf16x4 xf[4 * 64];                    // x^T: A operand of dW1
+    __shared__ float ypart[4][ROWS_PER_BLOCK];       // per column quarter
+    __shared__ float cols[3][4][H];                  // db1, db2, dW3 per row tile
+    __shared__ float sums[2][4];                     // db3 and loss per row tile
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int rt = wave & 3, cq = wave >> 2;         // row tile, column quarter (tiles 2 cq, 2 cq + 1)
     const bool train = a.t != nullptr;
-    for (int i = tid; i < H * H; i += 256) w2s[i] = a.w2b[i];
-    for (int i = tid; i < IN * H; i += 256) w1s[i] = a.w1b[i];
-    if (train) {
-        for (int i = tid; i < H * H; i += 256) gW2[i] = 0.f;
-        for (int i = tid; i < IN * H; i += 256) gW1[i] = 0.f;
-        for (int i = tid; i < 3 * H + 2; i += 256) gsmall[i] = 0.f;
-    }
-    __syncthreads();
+    const int lr = lane & 15, lg = lane >> 4;        // MFMA lane row/col and k group
+    const bf16x4 *F = reinterpret_cast<const bf16x4 *>(a.frag);
 
-    const int lr = lane & 15, lg = lane >> 4;  // MFMA lane row/col and k group
-    const unsigned row0 = blockIdx.x * ROWS_PER_BLOCK + wave * 16;
-    // the input row this lane loads for the A operand (row lr) and the D-layout rows 4*lg + j
-    auto src_row = [&](unsigned r) -> int {
-        const unsigned br = row0 + r;
-        if (br >= a.rows) return -1;
-        return (int)(a.sample ? pick_row(a.seed, a.step, br, a.n) : br);
-    };
-    const int ra = src_row(lr);
-    bf16x4 xa;
-    for (int j = 0; j < 4; ++j) xa[j] = ra >= 0 ? to_bf16(a.x[(size_t)ra * IN + 4 * lg + j]) : (short)0;
-
-    // ---- layer 1: z1 = x W1 + b1, h1 = tanh(z1); D layout: rows 4*lg + j, col 16*nt + lr
-    float h1[8][4];
-    for (int nt = 0; nt < 8; ++nt) {
-        bf16x4 bw;
-        for (int j = 0; j < 4; ++j) bw[j] = w1s[(4 * lg + j) * H + 16 * nt + lr];
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-        acc = mfma(xa, bw, acc);
-        const float bias = a.p[OFF_B1 + 16 * nt + lr];
-        for (int j = 0; j < 4; ++j) h1[nt][j] = tanhf(acc[j] + bias);
-    }
-    // re-layout h1 (BF16) through LDS into the A operand of layer 2
-    short *sc = scratch[wave];
-    for (int nt = 0; nt < 8; ++nt)
-        for (int j = 0; j < 4; ++j) sc[(4 * lg + j) * H + 16 * nt + lr] = to_bf16(h1[nt][j]);
-    __syncthreads();
-    // ---- layer 2
-    float h2[8][4];
-    for (int nt = 0; nt < 8; ++nt) {
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    // operand fragments of this wavefront's columns
+    bf16x4 w1f[2], w2f[2][8], w2t[2][8];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int nt = 2 * cq + i;
+        w1f[i] = F[FR_W1 / 4 + nt * 64 + lane];
+#pragma unroll
         for (int kt = 0; kt < 8; ++kt) {
-            bf16x4 av, bw;
-            for (int j = 0; j < 4; ++j) {
-                av[j] = sc[lr * H + 16 * kt + 4 * lg + j];
-                bw[j] = w2s[(16 * kt + 4 * lg + j) * H + 16 * nt + lr];
-            }
-            acc = mfma(av, bw, acc);
+            w2f[i][kt] = F[FR_W2 / 4 + (nt * 8 + kt) * 64 + lane];
+            if (train) w2t[i][kt] = F[FR_W2T / 4 + (nt * 8 + kt) * 64 + lane];
         }
-        const float bias = a.p[OFF_B2 + 16 * nt + lr];
-        for (int j = 0; j < 4; ++j) h2[nt][j] = tanhf(acc[j] + bias);
     }
-    // ---- layer 3: y[r] = h2[r] . W3 + b3; reduce over the 16 lanes of a k group
-    float yr[4];
-    for (int j = 0; j < 4; ++j) {
-        float s = 0.f;
-        for (int nt = 0; nt < 8; ++nt) s += h2[nt][j] * a.p[OFF_W3 + 16 * nt + lr];
-        for (int off = 8; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-        yr[j] = s + a.p[OFF_B3];
-    }
+    // the input row of lane row lr, and those of the D-layout rows 4 lg + j
+    const unsigned row0 = blockIdx.x * ROWS_PER_BLOCK + rt * 16;
+    int ra = -1;
+    if (row0 + lr < a.rows) ra = (int)(a.sample ? pick_row(a.seed, a.step, row0 + lr, a.n) : row0 + lr);
+    f32x4 xv = {0.f, 0.f, 0.f, 0.f};
+    if (ra >= 0) xv = *reinterpret_cast<const f32x4 *>(a.x + (size_t)ra * IN + 4 * lg);
     int rd[4];
-    for (int j = 0; j < 4; ++j) rd[j] = src_row(4 * lg + j);
-    if (a.y && lr == 0)
-        for (int j = 0; j < 4; ++j)
-            if (row0 + 4 * lg + j < a.rows) a.y[row0 + 4 * lg + j] = yr[j];
+    float tv[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        rd[j] = __shfl(ra, 4 * lg + j, 64);
+        tv[j] = train && rd[j] >= 0 ? a.t[rd[j]] : 0.f;
+    }
+    bf16x4 xa;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) xa[j] = to_bf16(xv[j]);
+    if (train && cq == 0) {
+        // x[row lr][4 lg + j] is element (k = 4 lg + j, row lr) of x^T: lane
+        // (lr / 4) * 16 + k, register lr % 4 of its A operand
+        short *xs = reinterpret_cast<short *>(xf + rt * 64);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) xs[((lr >> 2) * 16 + 4 * lg + j) * 4 + (lr & 3)] = xa[j];
+    }
+
+    // ---- layer 1: h1 = tanh(x W1 + b1)
+    float h1[2][4];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int nt = 2 * cq + i;
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        acc = mfma(xa, w1f[i], acc);
+        const float bias = a.p[OFF_B1 + 16 * nt + lr];
+        bf16x4 f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            h1[i][j] = tanhf(acc[j] + bias);
+            f[j] = to_bf16(h1[i][j]);
+            rows_lds[(rt * 16 + 4 * lg + j) * LD + 16 * nt + lr] = f[j];
+        }
+        h1f[(rt * 8 + nt) * 64 + lane] = f;
+    }
+    __syncthreads();
+    // ---- layer 2: h2 = tanh(h1 W2 + b2)
+    const short *arow = rows_lds + (rt * 16 + lr) * LD + 4 * lg;
+    float h2[2][4], w3[2];
+    {
+        f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int kt = 0; kt < 8; ++kt) {
+            const bf16x4 av = *reinterpret_cast<const bf16x4 *>(arow + 16 * kt);
+#pragma unroll
+            for (int i = 0; i < 2; ++i) acc[i] = mfma(av, w2f[i][kt], acc[i]);
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int c = 16 * (2 * cq + i) + lr;
+            const float bias = a.p[OFF_B2 + c];
+            w3[i] = a.p[OFF_W3 + c];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) h2[i][j] = tanhf(acc[i][j] + bias);
+        }
+    }
+    // ---- layer 3: y[r] = h2[r] . W3 + b3, over the 16 lanes of a k group and the four quarters
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        float s = h2[0][j] * w3[0] + h2[1][j] * w3[1];
+#pragma unroll
+        for (int off = 8; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+        if (lr == 0) ypart[cq][rt * 16 + 4 * lg + j] = s;
+    }
+    __syncthreads();
+    float yr[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int r = rt * 16 + 4 * lg + j;
+        yr[j] = ((ypart[0][r] + ypart[1][r]) + (ypart[2][r] + ypart[3][r])) + a.p[OFF_B3];
+        if (a.y && cq == 0 && lr == 0 && row0 + 4 * lg + j < a.rows) a.y[row0 + 4 * lg + j] = yr[j];
+    }
     if (!train) return;
 
     // ---- loss and dy = 2 (y - t) / rows (rows beyond the batch contribute 0)
-    float dy[4];
-    float lsum = 0.f;
+    float dy[4], dsum = 0.f, lsum = 0.f;
+#pragma unroll
     for (int j = 0; j < 4; ++j) {
-        if (rd[j] >= 0) {
-            const float e = yr[j] - a.t[rd[j]];
-            dy[j] = 2.f * e / (float)a.rows;
-            lsum += e * e;
-        } else {
-            dy[j] = 0.f;
-        }
+        const float e = rd[j] >= 0 ? yr[j] - tv[j] : 0.f;
+        dy[j] = 2.f * e / (float)a.rows;
+        dsum += dy[j];
+        lsum += e * e;
     }
-    // ---- dz2 = dy W3 (1 - h2^2); dW3 += dy h2; db2 += dz2
-    float dz2[8][4];
-    for (int nt = 0; nt < 8; ++nt) {
-        const float w3 = a.p[OFF_W3 + 16 * nt + lr];
+    dsum = col_sum(dsum);
+    lsum = col_sum(lsum);
+    if (cq == 0 && lane == 0) {
+        sums[0][rt] = dsum;
+        sums[1][rt] = lsum;
+    }
+    // ---- dz2 = dy W3 (1 - h2^2); dW3 = sum dy h2; db2 = sum dz2
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int nt = 2 * cq + i, c = 16 * nt + lr;
         float gw3 = 0.f, gb2 = 0.f;
+        bf16x4 f;
+#pragma unroll
         for (int j = 0; j < 4; ++j) {
-            dz2[nt][j] = dy[j] * w3 * (1.f - h2[nt][j] * h2[nt][j]);
-            gw3 += dy[j] * h2[nt][j];
-            gb2 += dz2[nt][j];
+            const float dz = dy[j] * w3[i] * (1.f - h2[i][j] * h2[i][j]);
+            gw3 += dy[j] * h2[i][j];
+            gb2 += dz;
+            f[j] = to_bf16(dz);
+            rows_lds[(rt * 16 + 4 * lg + j) * LD + c] = f[j];  // h1's rows were read before the last barrier
         }
-        atomicAdd(&gsmall[2 * H + 16 * nt + lr], gw3);
-        atomicAdd(&gsmall[H + 16 * nt + lr], gb2);
+        dzf[(rt * 8 + nt) * 64 + lane] = f;
+        gw3 = col_sum(gw3);
+        gb2 = col_sum(gb2);
+        if (lg == 0) {
+            cols[2][rt][c] = gw3;
+            cols[1][rt][c] = gb2;
+        }
     }
-    if (lr == 0) {
-        atomicAdd(&gsmall[3 * H], dy[0] + dy[1] + dy[2] + dy[3]);
-        atomicAdd(&gsmall[3 * H + 1], lsum);
-    }
-    // ---- dW2[k][c] += sum_r h1[r][k] dz2[r][c]: A = h1^T (D tile of h1), B = dz2 (D tile)
-    bf16x4 h1b[8], dzb[8];
-    for (int t8 = 0; t8 < 8; ++t8)
-        for (int j = 0; j < 4; ++j) {
-            h1b[t8][j] = to_bf16(h1[t8][j]);
-            dzb[t8][j] = to_bf16(dz2[t8][j]);
-        }
-    for (int mt = 0; mt < 8; ++mt)
-        for (int ct = 0; ct < 8; ++ct) {
-            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-            acc = mfma(h1b[mt], dzb[ct], acc);
-            for (int j = 0; j < 4; ++j) atomicAdd(&gW2[(16 * mt + 4 * lg + j) * H + 16 * ct + lr], acc[j]);
-        }
-    // ---- dh1 = dz2 W2^T: A = dz2 (re-laid through LDS), B[c][k] = W2[k][c]
-    __syncthreads();  // every wave is done reading its h1 scratch tile
-    for (int nt = 0; nt < 8; ++nt)
-        for (int j = 0; j < 4; ++j) sc[(4 * lg + j) * H + 16 * nt + lr] = dzb[nt][j];
     __syncthreads();
-    float dz1[8][4];
-    for (int nt = 0; nt < 8; ++nt) {
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    float *dst = a.partial + (size_t)blockIdx.x * PK;
+    // ---- dW2[k][c] = sum_r h1[r][k] dz2[r][c]: A = h1^T (D tiles of h1), B = dz2 (D tiles);
+    // row of tiles wave / 2, four of its tiles
+    {
+        const int mt = wave >> 1, c0 = (wave & 1) * 4;
+        f32x4 acc[4] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const bf16x4 av = h1f[(r * 8 + mt) * 64 + lane];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[i] = mfma(av, dzf[(r * 8 + c0 + i) * 64 + lane], acc[i]);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            *reinterpret_cast<f32x4 *>(dst + PK_W2 + ((mt * 8 + c0 + i) * 64 + lane) * 4) = acc[i];
+    }
+    // ---- dh1 = dz2 W2^T, dz1 = dh1 (1 - h1^2); db1 = sum dz1
+    bf16x4 d1[2];
+    {
+        f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
         for (int kt = 0; kt < 8; ++kt) {
-            bf16x4 av, bw;
+            const bf16x4 av = *reinterpret_cast<const bf16x4 *>(arow + 16 * kt);
+#pragma unroll
+            for (int i = 0; i < 2; ++i) acc[i] = mfma(av, w2t[i][kt], acc[i]);
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            float gb1 = 0.f;
+#pragma unroll
             for (int j = 0; j < 4; ++j) {
-                av[j] = sc[lr * H + 16 * kt + 4 * lg + j];
-                bw[j] = w2s[(16 * nt + lr) * H + 16 * kt + 4 * lg + j];
+                const float dz = acc[i][j] * (1.f - h1[i][j] * h1[i][j]);
+                gb1 += dz;
+                d1[i][j] = to_bf16(dz);
             }
-            acc = mfma(av, bw, acc);
+            gb1 = col_sum(gb1);
+            if (lg == 0) cols[0][rt][16 * (2 * cq + i) + lr] = gb1;
         }
-        float gb1 = 0.f;
-        for (int j = 0; j < 4; ++j) {
-            dz1[nt][j] = acc[j] * (1.f - h1[nt][j] * h1[nt][j]);
-            gb1 += dz1[nt][j];
-        }
-        atomicAdd(&gsmall[16 * nt + lr], gb1);
     }
-    // ---- dW1[k][c] += sum_r x[r][k] dz1[r][c]: A = x^T (lane rows 4 lg + j, k = lr)
-    bf16x4 xt;
-    for (int j = 0; j < 4; ++j) xt[j] = rd[j] >= 0 ? to_bf16(a.x[(size_t)rd[j] * IN + lr]) : (short)0;
-    for (int ct = 0; ct < 8; ++ct) {
-        bf16x4 bz;
-        for (int j = 0; j < 4; ++j) bz[j] = to_bf16(dz1[ct][j]);
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-        acc = mfma(xt, bz, acc);
-        for (int j = 0; j < 4; ++j) atomicAdd(&gW1[(4 * lg + j) * H + 16 * ct + lr], acc[j]);
-    }
+    __syncthreads();  // dz2's fragments are read
+#pragma unroll
+    for (int i = 0; i < 2; ++i) dzf[(rt * 8 + 2 * cq + i) * 64 + lane] = d1[i];
     __syncthreads();
-    float *dst = a.partial + (size_t)blockIdx.x * (NPARAM + 1);
-    for (int i = tid; i < IN * H; i += 256) dst[OFF_W1 + i] = gW1[i];
-    for (int i = tid; i < H * H; i += 256) dst[OFF_W2 + i] = gW2[i];
-    for (int i = tid; i < H; i += 256) {
-        dst[OFF_B1 + i] = gsmall[i];
-        dst[OFF_B2 + i] = gsmall[H + i];
-        dst[OFF_W3 + i] = gsmall[2 * H + i];
-    }
-    if (tid == 0) {
-        dst[OFF_B3] = gsmall[3 * H];
-        dst[NPARAM] = gsmall[3 * H + 1];
+    // ---- dW1[k][c] = sum_r x[r][k] dz1[r][c]
+    if (wave < 8) {
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc = mfma(xf[r * 64 + lane], dzf[(r * 8 + wave) * 64 + lane], acc);
+        *reinterpret_cast<f32x4 *>(dst + PK_W1 + (wave * 64 + lane) * 4) = acc;
+    } else {
+        const int i = tid - 512;
+        if (i < 3 * H) {
+            const int q = i / H, c = i % H;
+            dst[PK_B1 + i] = (cols[q][0][c] + cols[q][1][c]) + (cols[q][2][c] + cols[q][3][c]);
+        } else if (i < 3 * H + 2) {
+            const int q = i - 3 * H;
+            dst[PK_B3 + q] = (sums[q][0] + sums[q][1]) + (sums[q][2] + sums[q][3]);
+        }
     }
 }
 
-// Sums the block partials (fixed order) into grad, and optionally applies
-// one Adam step to the FP32 parameters and refreshes the BF16 copies.
-__global__ __launch_bounds__(256) void mlp_reduce_adam_kernel(const float *__restrict__ partial, int blocks,
-                                                              float *__restrict__ grad, float *__restrict__ loss,
-                                                              float *__restrict__ p, float *__restrict__ m,
-                                                              float *__restrict__ v, short *__restrict__ w1b,
-                                                              short *__restrict__ w2b, int apply, float lr,
-                                                              float b1c, float b2c) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i > NPARAM) return;
-    float g = 0.f;
-    for (int b = 0; b < blocks; ++b) g += partial[(size_t)b * (NPARAM + 1) + i];
-    if (i == NPARAM) {
-        if (loss) *loss = g;
+// The parameter of entry e of a workgroup's gradients (e < PK_LOSS).
+__device__ __forceinline__ int packed_param(int e) {
+    if (e >= PK_B1) {
+        const int q = e - PK_B1;
+        return q < H ? OFF_B1 + q : q < 2 * H ? OFF_B2 + q - H : q < 3 * H ? OFF_W3 + q - 2 * H : OFF_B3;
+    }
+    const bool second = e < PK_W1;
+    const int r = second ? e : e - PK_W1, tile = r >> 8, lane = (r >> 2) & 63, j = r & 3;
+    const int row = (second ? 16 * (tile >> 3) : 0) + 4 * (lane >> 4) + j, col = 16 * (tile & 7) + (lane & 15);
+    return (second ? OFF_W2 : OFF_W1) + row * H + col;
+}
+
+// The BF16 operand fragments of parameter i (of W1 or W2) with value v.
+__device__ __forceinline__ void put_fragment(short *frag, int i, float v) {
+    const short b = to_bf16(v);
+    if (i >= OFF_W1 && i < OFF_B1) {
+        const int k = (i - OFF_W1) / H, n = (i - OFF_W1) % H;
+        frag[FR_W1 + (((n >> 4) * 64) + (k >> 2) * 16 + (n & 15)) * 4 + (k & 3)] = b;
+    } else if (i >= OFF_W2 && i < OFF_B2) {
+        const int k = (i - OFF_W2) / H, n = (i - OFF_W2) % H;
+        frag[FR_W2 + (((n >> 4) * 8 + (k >> 4)) * 64 + ((k >> 2) & 3) * 16 + (n & 15)) * 4 + (k & 3)] = b;
+        frag[FR_W2T + (((k >> 4) * 8 + (n >> 4)) * 64 + ((n >> 2) & 3) * 16 + (k & 15)) * 4 + (n & 3)] = b;
+    }
+}
+
+// Sums the workgroups' gradients (fixed order) into grad, and optionally
+// applies one Adam step to the FP32 parameters and refreshes the BF16
+// fragments.  A thread takes 4 entries of every kSlices-th workgroup; the
+// slices meet in LDS.
+constexpr int kSlices = 16, kGroups = 16;
+__global__ __launch_bounds__(kSlices *kGroups) void mlp_reduce_adam_kernel(
+    const float *__restrict__ partial, int blocks, float *__restrict__ grad, float *__restrict__ loss,
+    float *__restrict__ p, float *__restrict__ m, float *__restrict__ v, short *__restrict__ frag, int apply, float lr,
+    float b1c, float b2c) {
+    __shared__ f32x4 sh[kSlices][kGroups];
+    const int g = threadIdx.x % kGroups, sl = threadIdx.x / kGroups;
+    const int e0 = ((int)blockIdx.x * kGroups + g) * 4;
+    f32x4 s = {0.f, 0.f, 0.f, 0.f};
+    if (e0 < PK) {
+#pragma unroll 4
+        for (int b = sl; b < blocks; b += kSlices) s += *reinterpret_cast<const f32x4 *>(partial + (size_t)b * PK + e0);
+    }
+    sh[sl][g] = s;
+    __syncthreads();
+    if (threadIdx.x >= kGroups * 4) return;
+    // one entry a thread
+    const int gi = threadIdx.x >> 2, j = threadIdx.x & 3, e = ((int)blockIdx.x * kGroups + gi) * 4 + j;
+    float gr = 0.f;
+    for (int k = 0; k < kSlices; ++k) gr += sh[k][gi][j];
+    if (e > PK_LOSS) return;
+    if (e == PK_LOSS) {
+        if (loss) *loss = gr;
         return;
     }
-    grad[i] = g;
+    const int i = packed_param(e);
+    grad[i] = gr;
     if (!apply) return;
     const float beta1 = 0.9f, beta2 = 0.999f, eps = 1e-8f;
-    const float mi = beta1 * m[i] + (1.f - beta1) * g;
-    const float vi = beta2 * v[i] + (1.f - beta2) * g * g;
+    const float mi = beta1 * m[i] + (1.f - beta1) * gr;
+    const float vi = beta2 * v[i] + (1.f - beta2) * gr * gr;
     m[i] = mi;
     v[i] = vi;
     const float pi = p[i] - lr * (mi / b1c) / (sqrtf(vi / b2c) + eps);
     p[i] = pi;
-    if (i >= OFF_W1 && i < OFF_B1) w1b[i - OFF_W1] = to_bf16(pi);
-    if (i >= OFF_W2 && i < OFF_B2) w2b[i - OFF_W2] = to_bf16(pi);
+    put_fragment(frag, i, pi);
 }
 
-__global__ void mlp_refresh_bf16_kernel(const float *__restrict__ p, short *__restrict__ w1b, short *__restrict__ w2b) {
+__global__ void mlp_fragments_kernel(const float *__restrict__ p, short *__restrict__ frag) {
     const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i < IN * H) w1b[i] = to_bf16(p[OFF_W1 + i]);
-    if (i < H * H) w2b[i] = to_bf16(p[OFF_W2 + i]);
+    if (i < NPARAM) put_fragment(frag, i, p[i]);
 }
 
 }  // namespace sxm
@@ -279,7 +383,7 @@ struct sx_mlp {
     std::string err;
     hipStream_t stream = nullptr;
     float *p = nullptr, *m = nullptr, *v = nullptr, *grad = nullptr, *partial = nullptr, *loss = nullptr;
-    short *w1b = nullptr, *w2b = nullptr;
+    short *frag = nullptr;
     float *x = nullptr, *t = nullptr, *y = nullptr;
     size_t xcap = 0, pcap_blocks = 0;
     unsigned long long adam_t = 0;
@@ -323,7 +427,7 @@ int ensure_partials(sx_mlp *n, size_t blocks) {
     if (blocks <= n->pcap_blocks) return SX_OK;
     if (n->partial) (void)hipFree(n->partial);
     n->partial = nullptr;
-    SXM_HIP(n, hipMalloc(&n->partial, sizeof(float) * (sxm::NPARAM + 1) * blocks));
+    SXM_HIP(n, hipMalloc(&n->partial, sizeof(float) * sxm::PK * blocks));
     n->pcap_blocks = blocks;
     return SX_OK;
 }
@@ -352,12 +456,11 @@ int step(sx_mlp *n, unsigned nrows_avail, unsigned rows, int sample, unsigned lo
     a.sample = sample;
     a.seed = seed;
     a.step = stepno;
-    a.w1b = n->w1b;
-    a.w2b = n->w2b;
+    a.frag = n->frag;
     a.p = n->p;
     a.y = train ? nullptr : n->y;
     a.partial = n->partial;
-    hipLaunchKernelGGL(sxm::mlp_step_kernel, dim3(blocks), dim3(256), 0, n->stream, a);
+    hipLaunchKernelGGL(sxm::mlp_step_kernel, dim3(blocks), dim3(sxm::kStepThreads), 0, n->stream, a);
     SXM_HIP(n, hipGetLastError());
     if (train) {
         float b1c = 1.f, b2c = 1.f;
@@ -366,9 +469,10 @@ int step(sx_mlp *n, unsigned nrows_avail, unsigned rows, int sample, unsigned lo
             b1c = 1.f - powf(0.9f, (float)n->adam_t);
             b2c = 1.f - powf(0.999f, (float)n->adam_t);
         }
-        hipLaunchKernelGGL(sxm::mlp_reduce_adam_kernel, dim3((sxm::NPARAM + 1 + 255) / 256), dim3(256), 0, n->stream,
-                           n->partial, (int)blocks, n->grad, n->loss, n->p, n->m, n->v, n->w1b, n->w2b, apply, lr,
-                           b1c, b2c);
+        constexpr int per = 4 * sxm::kGroups;
+        hipLaunchKernelGGL(sxm::mlp_reduce_adam_kernel, dim3((sxm::PK + per - 1) / per),
+                           dim3(sxm::kSlices * sxm::kGroups), 0, n->stream, n->partial, (int)blocks, n->grad, n->loss,
+                           n->p, n->m, n->v, n->frag, apply, lr, b1c, b2c);
         SXM_HIP(n, hipGetLastError());
     }
     return SX_OK;
@@ -401,8 +505,7 @@ int sx_mlp_create(int device, unsigned long long seed, sx_mlp **out) {
     fail(hipMalloc(&n->v, sizeof(float) * sxm::NPARAM));
     fail(hipMalloc(&n->grad, sizeof(float) * sxm::NPARAM));
     fail(hipMalloc(&n->loss, sizeof(float)));
-    fail(hipMalloc(&n->w1b, sizeof(short) * sxm::IN * sxm::H));
-    fail(hipMalloc(&n->w2b, sizeof(short) * sxm::H * sxm::H));
+    fail(hipMalloc(&n->frag, sizeof(short) * sxm::FR));
     if (rc != SX_OK) {
         sx_mlp_destroy(n);
         return rc;
@@ -434,8 +537,7 @@ void sx_mlp_destroy(sx_mlp *n) {
     if (n->stream) (void)hipStreamSynchronize(n->stream);
     for (float *q : {n->p, n->m, n->v, n->grad, n->partial, n->loss, n->x, n->t, n->y})
         if (q) (void)hipFree(q);
-    if (n->w1b) (void)hipFree(n->w1b);
-    if (n->w2b) (void)hipFree(n->w2b);
+    if (n->frag) (void)hipFree(n->frag);
     if (n->stream) (void)hipStreamDestroy(n->stream);
     delete n;
 }
@@ -447,8 +549,8 @@ int sx_mlp_set_params(sx_mlp *n, const float *params, size_t count) {
     SXM_HIP(n, hipMemcpyAsync(n->p, params, sizeof(float) * sxm::NPARAM, hipMemcpyHostToDevice, n->stream));
     SXM_HIP(n, hipMemsetAsync(n->m, 0, sizeof(float) * sxm::NPARAM, n->stream));
     SXM_HIP(n, hipMemsetAsync(n->v, 0, sizeof(float) * sxm::NPARAM, n->stream));
-    hipLaunchKernelGGL(sxm::mlp_refresh_bf16_kernel, dim3((sxm::H * sxm::H + 255) / 256), dim3(256), 0, n->stream,
-                       n->p, n->w1b, n->w2b);
+    hipLaunchKernelGGL(sxm::mlp_fragments_kernel, dim3((sxm::NPARAM + 255) / 256), dim3(256), 0, n->stream, n->p,
+                       n->frag);
     SXM_HIP(n, hipGetLastError());
     SXM_HIP(n, hipStreamSynchronize(n->stream));
     n->adam_t = 0;
