@@ -424,14 +424,15 @@ hipError_t launch_amp_oriented(const OrientArgs &a, hipStream_t stream) {
 
 // ------------------------------------------------------- few frames ------
 
-// pack[t][j] = (x, y, z, b) of atom j at frame t < NF; padding atoms as staged.
+// pack[t][j] = (x, y, z, b) of atom j at frame t < NF (b: one factor per atom,
+// or nullptr); padding atoms as staged.
 __global__ __launch_bounds__(256) void pack_frames_kernel(const float *__restrict__ X, const float *__restrict__ Y,
                                                           const float *__restrict__ Z, const float *__restrict__ b,
                                                           size_t NAp, size_t NFp, float4 *__restrict__ pack) {
     const size_t j = (size_t)blockIdx.x * 256 + threadIdx.x, t = blockIdx.y;
     if (j >= NAp) return;
     const size_t e = j * NFp + t;
-    pack[t * NAp + j] = make_float4(X[e], Y[e], Z[e], b[j]);
+    pack[t * NAp + j] = make_float4(X[e], Y[e], Z[e], b ? b[j] : 0.f);
 }
 
 // Work of a wavefront of the few-frames launch, items in the order
@@ -533,7 +534,7 @@ hipError_t launch_amp_few(const OrientArgs &a, int NF, int sub, float4 *pack, do
     k.sub = sub;
     k.NF = NF;
     hipLaunchKernelGGL(pack_frames_kernel, dim3((unsigned)((a.NAp + 255) / 256), (unsigned)NF), dim3(256), 0, stream,
-                       k.X, k.Y, k.Z, a.b, a.NAp, a.NFp, pack);
+                       k.X, k.Y, k.Z, a.per_shell_b ? nullptr : a.b, a.NAp, a.NFp, pack);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     const size_t items = (size_t)NF * a.split * sub * k.sgroups * k.ogroups;

@@ -11,8 +11,8 @@ struct OrientKernelArgs {
     size_t NFp;
     const double *qlen;    // [ns] |q_s| / 2 pi
     const double *u;       // [NM][3] unit orientations
-    const float *b;        // [nb][NAp]
-    size_t NAp;            // row stride of the coordinate planes and of b
+    const float *b;        // [NAp], or one factor per shell and atom: [NAp][ns] and kWave floats more
+    size_t NAp;            // row stride of the coordinate planes
     size_t natoms;         // atoms summed (<= NAp)
     int NM, ns, V, ftiles, ogroups, sgroups, split, atoms_per_split, per_shell_b;
     float2 *amp;           // [split][V][NFp], v = s * NM + m
@@ -220,7 +220,8 @@ __device__ __forceinline__ void oriented_tile_body(const OrientKernelArgs &a, in
                 float bk[VS];
 #pragma unroll
                 for (int k = 0; k < VS; ++k)
-                    bk[k] = PER_ROW_B ? B[(size_t)min(sbase + k, a.ns - 1) * a.NAp + j + c] : LQ ? bs[LQ ? c : 0] : B[j + c];
+                    // (shells past the last read the next atom's factors; their sums are not kept)
+                    bk[k] = PER_ROW_B ? B[(j + c) * a.ns + sbase + k] : LQ ? bs[LQ ? c : 0] : B[j + c];
 #pragma unroll
                 for (int i = 0; i < VM; ++i) {
                     double d = ux[i] * xd;

@@ -430,14 +430,25 @@ int run_batch(sx_ctx *c, int ns, size_t NM, const double *qv, const double *qlen
     const float *bptr = c->b.as<float>();
     const int *browp = nullptr;
     if (b_shell) {
-        std::vector<float> bs((size_t)ns * c->NAp, 0.f);
-        for (int s = 0; s < ns; ++s)
-            for (size_t j = 0; j < c->NA; ++j) bs[(size_t)s * c->NAp + j] = (float)b_shell[(size_t)s * c->NA + j];
+        // rows of atoms per shell; the oriented coherent kernel reads the
+        // shells' factors of an atom together
+        const bool by_atom = oriented && !self;
+        std::vector<float> bs((size_t)ns * c->NAp + (by_atom ? sx::kShellFactorPad : 0), 0.f);
+        if (by_atom) {
+            for (size_t j0 = 0; j0 < c->NA; j0 += 16)
+                for (int s = 0; s < ns; ++s)
+                    for (size_t j = j0; j < std::min(c->NA, j0 + 16); ++j)
+                        bs[j * ns + s] = (float)b_shell[(size_t)s * c->NA + j];
+        } else {
+            for (int s = 0; s < ns; ++s)
+                for (size_t j = 0; j < c->NA; ++j)
+                    bs[(size_t)s * c->NAp + j] = (float)b_shell[(size_t)s * c->NA + j];
+        }
         SX_HIP(c, c->bshell.ensure(sizeof(float) * bs.size()));
         SX_HIP(c, hipMemcpyAsync(c->bshell.p, bs.data(), sizeof(float) * bs.size(), hipMemcpyHostToDevice,
                                  c->stream));
         bptr = c->bshell.as<float>();
-        if (!self) {
+        if (!self && !by_atom) {
             std::vector<int> br(V);
             for (int v = 0; v < V; ++v) br[v] = v / (int)NM;
             SX_HIP(c, c->brow.ensure(sizeof(int) * V));
@@ -1183,7 +1194,7 @@ size_t noalloc_batch_bytes(sx_ctx *c, int ns, const double *qlen, size_t NM, boo
         sizeof(double) * ns,                                      // qlen
         sizeof(double) * 3 * NM,                                  // uvec
         mode == 2 ? sx::shell_table_bytes(ns) : 0,                // qres (runs and residuals)
-        per_shell ? sizeof(float) * ns * c->NAp : 0,              // bshell
+        per_shell ? sizeof(float) * ns * c->NAp : 0,              // bshell (its 128 bytes behind: in the slack)
         per_shell ? sizeof(int) * V : 0,                          // brow
         sizeof(float2) * V * c->NFp * split,                      // amp
         sizeof(double) * 4 * ns * chunks,                         // apart

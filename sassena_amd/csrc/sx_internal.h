@@ -112,6 +112,8 @@ struct TileLine {
 };
 constexpr int kTileCorrectUp = 1, kTileCorrectDown = 2;
 
+constexpr size_t kShellFactorPad = 32;
+
 // Oriented shells: v = s * NM + m has q_v = |q_s| u_m.  NAp must be a multiple
 // of 16 (it is a multiple of 64).
 struct OrientArgs {
@@ -119,7 +121,11 @@ struct OrientArgs {
     size_t NAp, NFp;
     const double *qlen;    // [ns] |q_s| / 2 pi
     const double *u;       // [NM][3]
-    const float *b;        // [ns][NAp] if per_shell_b else [NAp]
+    // [NAp], or if per_shell_b [NAp][ns] with kShellFactorPad floats behind (the
+    // factors of a tile's shells are then one scalar load an atom; as rows of
+    // atoms they took the scalar registers of 16 atoms x 8 shells: 9.1 ms against
+    // 4.7 for 7,001 atoms x 1,501 frames x 21 shells x 67 orientations)
+    const float *b;
     int NM, ns, split, per_shell_b;
     int shape = 0;         // tile shape index (< kOrientShapes)
     float2 *amp;           // [split][ns*NM][NFp]
