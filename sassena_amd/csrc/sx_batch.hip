@@ -80,12 +80,12 @@ __global__ void reset_counters_kernel(unsigned *c, int n) {
     if (i < n) c[i] = 0u;
 }
 
-template <typename C, int NH, int E>
-__global__ __launch_bounds__(512) void corr_batch_kernel(const CorrArgs *__restrict__ cargs,
-                                                         const int4 *__restrict__ items) {
+template <typename PT, int E>
+__global__ __launch_bounds__(PT::T, corr_all_waves<E>()) void corr_batch_kernel(const CorrArgs *__restrict__ cargs,
+                                                           const int4 *__restrict__ items) {
     extern __shared__ double2 lds_d[];
     const int4 w = items[blockIdx.x];
-    corr_all_block<C, NH, E>(cargs[w.x], w.y, w.z, lds_d);
+    corr_all_block<PT, E>(cargs[w.x], w.y, w.z, lds_d);
 }
 
 __global__ __launch_bounds__(kFinalThreads) void final_reduce_batch_kernel(const FinalArgs *__restrict__ fargs,
@@ -138,15 +138,20 @@ static PersistentFn persistent_fn(int shape, int kind) {
     return kind == 2 ? persistent_fn_of<2>(shape) : kind == 1 ? persistent_fn_of<1>(shape) : persistent_fn_of<0>(shape);
 }
 
-static CorrBatchFn corr_batch_fn(int E) {
-    switch (E) {
-        case 4: return corr_batch_kernel<double2, 1, 4>;
-        case 8: return corr_batch_kernel<double2, 1, 8>;
-        case 16: return corr_batch_kernel<double2, 1, 16>;
-        case 20: return corr_batch_kernel<double2, 1, 20>;
-        case 24: return corr_batch_kernel<double2, 1, 24>;
-        default: return nullptr;
-    }
+static CorrBatchFn corr_batch_fn(const FftPlan &P) {
+    if (Plan256::matches(P)) return corr_batch_kernel<Plan256, 4>;
+    if (Plan512::matches(P)) return corr_batch_kernel<Plan512, 8>;
+    if (Plan1024::matches(P)) return corr_batch_kernel<Plan1024, 8>;
+    if (Plan1536::matches(P)) return corr_batch_kernel<Plan1536, 24>;
+    if (Plan2048::matches(P)) return corr_batch_kernel<Plan2048, 8>;
+    if (Plan2560::matches(P)) return corr_batch_kernel<Plan2560, 20>;
+    if (Plan3072::matches(P)) return corr_batch_kernel<Plan3072, 24>;
+    if (Plan4096::matches(P)) return corr_batch_kernel<Plan4096, 16>;
+    if (Plan5120::matches(P)) return corr_batch_kernel<Plan5120, 20>;
+    if (Plan6144::matches(P)) return corr_batch_kernel<Plan6144, 24>;
+    if (Plan8192::matches(P)) return corr_batch_kernel<Plan8192, 16>;
+    if (Plan10240::matches(P)) return corr_batch_kernel<Plan10240, 20>;
+    return nullptr;
 }
 
 }  // namespace sx
@@ -186,7 +191,8 @@ struct Plan {
     int nitems = 0, nritems = 0, nfitems = 0;
     size_t terms_exact_runs = 0;  // terms of mode-2 tiles stepped without corrections (kind 2)
     struct CorrGroup {
-        int E, T, first, count;
+        sx::FftPlan plan;
+        int first, count;
         size_t lds;
     };
     std::vector<CorrGroup> groups;
@@ -460,7 +466,7 @@ int build_plan(sx_batch *b, const std::vector<int> &ks, int shape, Plan &P) {
         const sx::FftPlan &pl = b->work[kv.second[0].x].ctx->plan;
         // corr_all_block reduces a_m in the start of the FFT buffer, so the
         // dynamic LDS is exactly the transform data (160 KB at Lh = 10240)
-        Plan::CorrGroup g{pl.E, pl.T, (int)citems.size(), (int)kv.second.size(), sx::corr_all_lds_bytes(pl)};
+        Plan::CorrGroup g{pl, (int)citems.size(), (int)kv.second.size(), sx::corr_all_lds_bytes(pl)};
         P.groups.push_back(g);
         citems.insert(citems.end(), kv.second.begin(), kv.second.end());
     }
@@ -496,9 +502,9 @@ int launch_amplitude(sx_batch *b, Plan &P) {
 
 int launch_rest(sx_batch *b, Plan &P) {
     for (const Plan::CorrGroup &g : P.groups) {
-        sx::CorrBatchFn fn = sx::corr_batch_fn(g.E);
-        if (!fn) return bfail(b, SX_ERR_UNSUPPORTED, "no correlation kernel for E=%d", g.E);
-        hipLaunchKernelGGL(fn, dim3(g.count), dim3(g.T), g.lds, b->stream, P.cargs.as<sx::CorrArgs>(),
+        sx::CorrBatchFn fn = sx::corr_batch_fn(g.plan);
+        if (!fn) return bfail(b, SX_ERR_UNSUPPORTED, "no correlation kernel for length %d", g.plan.Lh);
+        hipLaunchKernelGGL(fn, dim3(g.count), dim3(g.plan.T), g.lds, b->stream, P.cargs.as<sx::CorrArgs>(),
                            P.citems.as<int4>() + g.first);
         SXB_HIP(b, hipGetLastError());
     }
@@ -514,7 +520,7 @@ int launch_rest(sx_batch *b, Plan &P) {
 int capture(sx_batch *b, Plan &P) {
     // kernel attributes are set before capture (dynamic LDS above 64 KB)
     for (const Plan::CorrGroup &g : P.groups)
-        SXB_HIP(b, hipFuncSetAttribute((const void *)sx::corr_batch_fn(g.E),
+        SXB_HIP(b, hipFuncSetAttribute((const void *)sx::corr_batch_fn(g.plan),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)g.lds));
     hipGraph_t g = nullptr;
     SXB_HIP(b, hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));

@@ -101,10 +101,10 @@ bool make_fft_plan(size_t NF, FftPlan *plan) {
     return best && plan_from(*best, bestN1, plan);
 }
 
-template <typename C, int NH, int E>
-__global__ __launch_bounds__(512) void corr_all_kernel(CorrArgs a) {
+template <typename PT, int E>
+__global__ __launch_bounds__(PT::T, corr_all_waves<E>()) void corr_all_kernel(CorrArgs a) {
     extern __shared__ double2 lds_d[];
-    corr_all_block<C, NH, E>(a, blockIdx.x / a.chunks, blockIdx.x % a.chunks, lds_d);
+    corr_all_block<PT, E>(a, blockIdx.x / a.chunks, blockIdx.x % a.chunks, lds_d);
 }
 
 template <typename C, int NH, int E>
@@ -666,10 +666,30 @@ hipError_t launch_self_a_reduce(const double2 *apair, long npairs, int wpp, int 
     return hipGetLastError();
 }
 
+static CorrKernel corr_all_fn(const FftPlan &P) {
+    if (Plan256::matches(P)) return corr_all_kernel<Plan256, 4>;
+    if (Plan512::matches(P)) return corr_all_kernel<Plan512, 8>;
+    if (Plan1024::matches(P)) return corr_all_kernel<Plan1024, 8>;
+    if (Plan1536::matches(P)) return corr_all_kernel<Plan1536, 24>;
+    if (Plan2048::matches(P)) return corr_all_kernel<Plan2048, 8>;
+    if (Plan2560::matches(P)) return corr_all_kernel<Plan2560, 20>;
+    if (Plan3072::matches(P)) return corr_all_kernel<Plan3072, 24>;
+    if (Plan4096::matches(P)) return corr_all_kernel<Plan4096, 16>;
+    if (Plan5120::matches(P)) return corr_all_kernel<Plan5120, 20>;
+    if (Plan6144::matches(P)) return corr_all_kernel<Plan6144, 24>;
+    if (Plan8192::matches(P)) return corr_all_kernel<Plan8192, 16>;
+    if (Plan10240::matches(P)) return corr_all_kernel<Plan10240, 20>;
+    return nullptr;
+}
+
 hipError_t launch_corr_all(const CorrArgs &a, hipStream_t stream) {
-    return launch_corr<double2, 1>(corr_all_kernel<double2, 1, 4>, corr_all_kernel<double2, 1, 8>,
-                                   corr_all_kernel<double2, 1, 16>, corr_all_kernel<double2, 1, 20>,
-                                   corr_all_kernel<double2, 1, 24>, a, stream);
+    const CorrKernel k = corr_all_fn(a.plan);
+    if (!k) return hipErrorInvalidValue;
+    const size_t lds = corr_all_lds_bytes(a.plan);
+    hipError_t e = hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k, dim3((unsigned)(a.nshells * a.chunks)), dim3(a.plan.T), lds, stream, a);
+    return hipGetLastError();
 }
 
 hipError_t launch_corr_self(const CorrArgs &a, int halves, hipStream_t stream) {

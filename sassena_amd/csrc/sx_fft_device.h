@@ -427,11 +427,14 @@ __device__ __forceinline__ void spass_first(C (&v)[E], C *buf, const Input &in, 
 
 // The twiddles of the middle passes of a fixed plan for one thread: every
 // group of the thread has the index kk = ut mod Ns in pass p, so each pass
-// needs R - 1 of them, the same for every series; loaded once per kernel and
-// kept in registers.
+// needs R - 1 of them, the same for every series; in FP32 loaded once per
+// kernel and kept in registers (pass_twiddle).  In FP64 they would take up
+// to 72 registers for the few series of a block: loaded in each pass, ahead of
+// its barrier.
 template <typename C, typename PT>
 struct MidTwiddles {
-    C w[PT::npass][8];
+    static constexpr bool kKept = sizeof(C) == 8;
+    C w[kKept ? PT::npass : 1][8];
     const C *twp;  // the pass twiddle table (passes with Ns > T load theirs per series)
     template <int p>
     __device__ __forceinline__ void load_from(const C *__restrict__ twp, unsigned ut) {
@@ -447,7 +450,18 @@ struct MidTwiddles {
     }
     __device__ __forceinline__ void load(const C *__restrict__ tw, unsigned ut) {
         twp = tw;
-        load_from<1>(tw, ut);
+        if constexpr (kKept) load_from<1>(tw, ut);
+    }
+    // the twiddles of pass p (Ns <= T) into t
+    template <int p>
+    __device__ __forceinline__ void pass(C (&t)[8], unsigned ut) const {
+        constexpr int R = PT::radix(p);
+        const unsigned kk = ut & (PT::ns(p) - 1);
+#pragma unroll
+        for (int q = 1; q < R; ++q) {
+            if constexpr (kKept) t[q] = w[p][q];
+            else t[q] = twiddle_load(twp, kk * R, PT::toff(p) + q);
+        }
     }
 };
 
@@ -497,7 +511,8 @@ __device__ __forceinline__ void spass_mid(C (&v)[E], C *buf, const MidTwiddles<C
     } else {
         // every group of the thread has the twiddle index kk = ut mod Ns
         const unsigned kk = ut & (Ns - 1);
-        const C(&ws)[8] = mt.w[p];
+        C ws[8];
+        mt.template pass<p>(ws, ut);
         const unsigned rb = PT::swz(p - 1, ut);
 #pragma unroll
         for (int i = 0; i < E / R; ++i)
@@ -616,6 +631,8 @@ __device__ __forceinline__ void spass_last_fused(C (&v)[E], Acc (&acc)[2][E], co
     C base[RB];
 #pragma unroll
     for (int b = 1; b < RB; ++b) base[b] = twiddle_load(twp, ut * RB, PT::toff(pb) + b);
+    C wa[8];
+    mt.template pass<pa>(wa, ut);
     const unsigned rb = PT::swz(pa - 1, ut);
 #pragma unroll
     for (int q = 0; q < R; ++q) v[q] = buf[rb + q * T];
@@ -625,7 +642,7 @@ __device__ __forceinline__ void spass_last_fused(C (&v)[E], Acc (&acc)[2][E], co
 #pragma unroll
         for (int b = 0; b < RB; ++b) {
             if (a == 0 && b == 0) continue;
-            const C t = a == 0 ? base[b] : b == 0 ? mt.w[pa][a] : cmul(mt.w[pa][a], base[b]);
+            const C t = a == 0 ? base[b] : b == 0 ? wa[a] : cmul(wa[a], base[b]);
             v[RB * a + b] = cmul(v[RB * a + b], t);
         }
     C y[RA][RB];
@@ -658,13 +675,11 @@ __device__ __forceinline__ void spass_last_fused(C (&v)[E], Acc (&acc)[2][E], co
     }
 }
 
-// One half H of a padded series through the fixed plan PT.
-template <typename C, int E, typename PT, int H, typename Acc, typename Input>
-__device__ __forceinline__ void fft_sweep_fixed(C (&v)[E], Acc (&acc)[2][E], C *buf, const C *__restrict__ tw,
-                                                const MidTwiddles<C, PT> &mt, const double2 *__restrict__ w,
-                                                const Input &in, double &ar, double &ai, unsigned ut) {
-    static_assert(H == 0 || Input::kPretwiddled, "the odd-bin half needs its input pre-twiddled");
-    spass_first<C, E, PT>(v, buf, in, ut);
+// The passes after the first of one half H, the power spectrum into acc and a.
+template <typename C, int E, typename PT, int H, typename Acc>
+__device__ __forceinline__ void fft_sweep_rest(C (&v)[E], Acc (&acc)[2][E], C *buf, const C *__restrict__ tw,
+                                               const MidTwiddles<C, PT> &mt, const double2 *__restrict__ w, double &ar,
+                                               double &ai, unsigned ut) {
     if constexpr (fused_last<PT, E>()) {
         spass_mids<C, E, PT, 1, PT::npass - 2>(v, buf, mt, ut);
         spass_last_fused<C, E, PT, H>(v, acc, buf, tw, mt, w, ar, ai, ut);
@@ -672,6 +687,32 @@ __device__ __forceinline__ void fft_sweep_fixed(C (&v)[E], Acc (&acc)[2][E], C *
         spass_mids<C, E, PT, 1, PT::npass - 1>(v, buf, mt, ut);
         spass_last<C, E, PT, H>(v, acc, buf, tw, w, ar, ai, ut);
     }
+}
+
+// One half H of a padded series through the fixed plan PT.
+template <typename C, int E, typename PT, int H, typename Acc, typename Input>
+__device__ __forceinline__ void fft_sweep_fixed(C (&v)[E], Acc (&acc)[2][E], C *buf, const C *__restrict__ tw,
+                                                const MidTwiddles<C, PT> &mt, const double2 *__restrict__ w,
+                                                const Input &in, double &ar, double &ai, unsigned ut) {
+    static_assert(H == 0 || Input::kPretwiddled, "the odd-bin half needs its input pre-twiddled");
+    spass_first<C, E, PT>(v, buf, in, ut);
+    fft_sweep_rest<C, E, PT, H>(v, acc, buf, tw, mt, w, ar, ai, ut);
+}
+
+// The first pass from the points v[i R + q] = x(ut + i T + q Lh / R), then the rest.
+template <typename C, int E, typename PT, int H, typename Acc>
+__device__ __forceinline__ void fft_sweep_loaded(C (&v)[E], Acc (&acc)[2][E], C *buf, const C *__restrict__ tw,
+                                                 const MidTwiddles<C, PT> &mt, const double2 *__restrict__ w,
+                                                 double &ar, double &ai, unsigned ut) {
+    constexpr int R = PT::radix(0);
+#pragma unroll
+    for (int i = 0; i < E / R; ++i) {
+        Dft<R, C>::run(&v[i * R]);
+#pragma unroll
+        for (int q = 0; q < R; ++q) buf[PT::swz(0, ut * R + (q & ~1)) + (q & 1) + i * PT::T * R] = v[i * R + q];
+    }
+    __syncthreads();
+    fft_sweep_rest<C, E, PT, H>(v, acc, buf, tw, mt, w, ar, ai, ut);
 }
 
 // The one-block half-lengths of the self path (the runtime plans of
@@ -773,24 +814,6 @@ __device__ __forceinline__ void flush_power_half(const FftPlan &P, Acc (&acc)[2]
 constexpr int kFlushEvery = 16;
 
 template <typename C>
-struct AmpInput {
-    static constexpr bool kPretwiddled = false;
-    static constexpr bool kBounded = false;
-    const float2 *p;
-    size_t split_stride;
-    int split;
-    __device__ __forceinline__ C operator()(unsigned n) const {
-        float2 s = p[n];
-        for (int k = 1; k < split; ++k) {
-            const float2 t = p[(size_t)k * split_stride + n];
-            s.x += t.x;
-            s.y += t.y;
-        }
-        return Cx<C>::make(s.x, s.y);
-    }
-};
-
-template <typename C>
 __device__ __forceinline__ const C *pass_twiddles(const CorrArgs &a);
 template <>
 __device__ __forceinline__ const float2 *pass_twiddles<float2>(const CorrArgs &a) {
@@ -811,55 +834,93 @@ __device__ __forceinline__ const double2 *pre_twiddles<double2>(const CorrArgs &
     return a.twL64;
 }
 
+// Bounded for two wavefronts a SIMD where that leaves no more than a few
+// registers in scratch (16 points a thread; 20 and 24 spill over 100).
+template <int E>
+constexpr int corr_all_waves() {
+    return E == 16 ? 2 : 1;
+}
+
 // "all": one block per (shell, chunk of vectors); the series of vector v is
-// its coherent amplitude A_v(t) from HBM (sum of the atom-range partials).
-// One block of the coherent correlation: shell s, vector chunk c.
-template <typename C, int NH, int E>
-__device__ __forceinline__ void corr_all_block(const CorrArgs &a, int s, int c, double2 *lds_d) {
-    using Acc = typename Cx<C>::R;
-    C *buf = reinterpret_cast<C *>(lds_d);
+// its coherent amplitude A_v(t) from HBM (sum of the atom-range partials),
+// transformed in FP64 through the fixed plan of its length.  A thread loads its
+// points of a series once for both halves, all points of an atom range
+// in flight together (bounded buffer loads: 0 past the series), and adds the
+// ranges in FP32 in their order.  Bound by the latency of the passes for few
+// series, by LDS and registers for many.  Against the runtime plan with its
+// index arithmetic, points read per half and one range after the other: one
+// shell of 200 vectors x 2,000 frames 40 -> 18 us, 40 shells 595 -> 283 us, 50
+// vectors x 200 frames 18 -> 9 us, 1,000 x 6,000 frames 511 -> 262 us; 4,000 to
+// 5,000 frames gain 3 to 5 %, 10,000 nothing.
+template <typename PT, int E>
+__device__ __forceinline__ void corr_all_block(const CorrArgs &a, int s, int c, double2 *buf) {
     const FftPlan &P = a.plan;
     // The block reduction of a_m runs after the last pass has read the
     // buffer behind a barrier, and ends with a barrier before the next series
     // writes it, so it can use the start of the FFT buffer.
-    double2 *red = reinterpret_cast<double2 *>(buf);
-    const C *tw = pass_twiddles<C>(a);
-    const C *pre = pre_twiddles<C>(a);
+    double2 *red = buf;
     const int tid = threadIdx.x;
     const int m0 = (int)((long)a.NM * c / a.chunks), m1 = (int)((long)a.NM * (c + 1) / a.chunks);
+    constexpr int R = PT::radix(0);
+    constexpr unsigned T = PT::T, stride = PT::Lh / R;
+    // Registers of many points a thread: the points come again from L2 for the
+    // second half, or (512 threads: 256 registers each) the power goes to the
+    // row after each half.
+    constexpr bool kReload = E >= 16 && T <= 256, kFlush = E >= 20 && T > 256;
 
-    C v[NH][E];
-    Acc acc[2][E];
+    double2 v[E];
+    double acc[2][E];
 #pragma unroll
-    for (int e = 0; e < E; ++e) acc[0][e] = acc[1][e] = Acc(0);
+    for (int e = 0; e < E; ++e) acc[0][e] = acc[1][e] = 0.0;
     double sa_r = 0.0, sa_i = 0.0, sa2 = 0.0;
     double *row = a.ppart + ((size_t)s * a.chunks + c) * P.L;
-    const bool fp32 = sizeof(Acc) == 4;
-    bool first = true;
-    int since = 0;
+    MidTwiddles<double2, PT> mt;
+    mt.load(a.twp64, (unsigned)tid);
     for (int m = m0; m < m1; ++m) {
-        const size_t vidx = (size_t)s * a.NM + m;
-        AmpInput<C> in{a.amp + vidx * a.NFp, a.split_stride, a.split};
-        double ar = 0.0, ai = 0.0;
+        const float2 *p = a.amp + ((size_t)s * a.NM + m) * a.NFp;
         // Opaque copy of the thread index: keeps the compiler from hoisting
         // every pass's address arithmetic out of the series loop (which
         // would not fit in registers).
         int t = tid;
         asm volatile("" : "+v"(t));
-        fft_power<C, NH, E>(P, v, acc, buf, tw, pre, a.w, a.NF, in, ar, ai, t);
-        const double2 r = block_sum2(ar, ai, red, tid, P.T);
+        const unsigned ut = (unsigned)t;
+        float2 x[E];
+        auto load = [&]() {
+            for (int k = 0; k < a.split; ++k) {
+                const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+                    (void *)(p + (size_t)k * a.split_stride), (short)0, a.NF * 8, kBufferDword3);
+#pragma unroll
+                for (int e = 0; e < E; ++e) {
+                    const auto y =
+                        __builtin_amdgcn_raw_buffer_load_b64(r, (ut + (e / R) * T + (e % R) * stride) * 8u, 0, 0);
+                    const float yr = __uint_as_float(y[0]), yi = __uint_as_float(y[1]);
+                    x[e].x = k ? x[e].x + yr : yr;
+                    x[e].y = k ? x[e].y + yi : yi;
+                }
+            }
+        };
+        load();
+        double ar = 0.0, ai = 0.0;
+#pragma unroll
+        for (int e = 0; e < E; ++e) v[e] = make_double2(x[e].x, x[e].y);
+        fft_sweep_loaded<double2, E, PT, 0>(v, acc, buf, a.twp64, mt, a.w, ar, ai, ut);
+        if constexpr (kFlush) flush_power_half<E, 0>(P, acc, row, m == m0, tid);
+        if constexpr (kReload) load();
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            const double2 w = twiddle_load(a.twL64, ut, (e / R) * T + (e % R) * stride);
+            v[e] = cmul(make_double2(x[e].x, x[e].y), w);
+        }
+        fft_sweep_loaded<double2, E, PT, 1>(v, acc, buf, a.twp64, mt, a.w, ar, ai, ut);
+        if constexpr (kFlush) flush_power_half<E, 1>(P, acc, row, m == m0, tid);
+        const double2 r = block_sum2(ar, ai, red, tid, PT::T);
         if (tid == 0) {
             sa_r += r.x;
             sa_i += r.y;
             sa2 += r.x * r.x + r.y * r.y;
         }
-        if (fp32 && ++since == kFlushEvery) {
-            flush_power<E>(P, acc, row, first, tid);
-            first = false;
-            since = 0;
-        }
     }
-    if (since > 0 || first || !fp32) flush_power<E>(P, acc, row, first, tid);
+    if constexpr (!kFlush) flush_power<E>(P, acc, row, true, tid);
     if (tid == 0) {
         double *ap = a.apart + ((size_t)s * a.chunks + c) * 4;
         ap[0] = sa_r;
