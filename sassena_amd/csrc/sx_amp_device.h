@@ -40,9 +40,8 @@ constexpr size_t kResidualLds = sizeof(double) * 4 * VM * VS * 2 * kWave;
 
 OrientKernelArgs make_orient_args(const OrientArgs &a);
 
-// One tile of the oriented amplitude sum: frame tile ft (one frame per
-// lane), atom range sp, orientations 4*VM*og.. (VM per wavefront) and
-// shells sbase..sbase+VS-1; 256 threads.  MODE 1: the shells of the call are in
+// One wavefront's tile of the oriented amplitude sum: frame tile ft (one frame
+// per lane), atom range sp, orientations VM*og.. and shells sbase..sbase+VS-1.  MODE 1: the shells of the call are in
 // arithmetic progression (step a.qstep), and the tile's shells follow from its
 // middle one by the three-term recurrence.  MODE 2: as 1 on the ideal grid
 // q0 + s qstep, with each shell's residual r_s = q_s - (q0 + s qstep) (the
@@ -99,7 +98,7 @@ __device__ __forceinline__ void oriented_tile_body(const OrientKernelArgs &a, in
     constexpr int kFold = 64;  // atoms per FP32 partial sum
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
-    const int mbase = LQ ? og * kWave + lane : (og * 4 + wave) * VM;
+    const int mbase = LQ ? og * kWave + lane : og * VM;
     const size_t t = LQ ? (size_t)ft : (size_t)ft * kWave + lane;
 
     const auto U = uniform_ptr(a.u);

@@ -66,12 +66,13 @@ __global__ __launch_bounds__(256, 2) void amp_persistent_kernel(const OrientKern
         __syncthreads();  // every thread has read cur before it is overwritten
         if (it >= n) break;
         const int4 w = items[begin + it];
+        const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
         if constexpr (KIND == 1)
-            oriented_tile_body<VM, VS, false, 2, true>(targs[w.x], w.y, 0, w.z & 0xffff, w.z >> 16, tot_lds);
+            oriented_tile_body<VM, VS, false, 2, true>(targs[w.x], w.y, 0, (w.z & 0xffff) * 4 + wave, w.z >> 16, tot_lds);
         else if constexpr (KIND == 2)
-            oriented_tile_body<VM, VS, false, 3, true>(targs[w.x], w.y, 0, w.z & 0xffff, w.z >> 16, tot_lds);
+            oriented_tile_body<VM, VS, false, 3, true>(targs[w.x], w.y, 0, (w.z & 0xffff) * 4 + wave, w.z >> 16, tot_lds);
         else
-            oriented_tile<VM, VS, false, false>(targs[w.x], w.y, 0, w.z & 0xffff, w.z >> 16);
+            oriented_tile<VM, VS, false, false>(targs[w.x], w.y, 0, (w.z & 0xffff) * 4 + wave, w.z >> 16);
     }
 }
 
@@ -326,7 +327,7 @@ int build_plan(sx_batch *b, const std::vector<int> &ks, int shape, Plan &P) {
         const sx_trajectory &t = b->trajs[k];
         const bool res = b->work[k].mode == 2;
         oka[k] = orient_args(b->work[k], t, args_shape);
-        const int ftiles = oka[k].ftiles, og = oka[k].ogroups;
+        const int ftiles = oka[k].ftiles, og = (oka[k].ogroups + 3) / 4;  // a workgroup: four wavefronts
         std::vector<ShellGroup> groups;
         if (mixed) {
             groups = shell_groups((int)t.nshells, res);
