@@ -619,6 +619,9 @@ int sx_batch_stage(sx_batch *b, const sx_trajectory *trajs, size_t ntraj) {
         int rc = sx_create(&c, &w.ctx);
         if (rc != SX_OK) return bfail(b, rc, "trajectory %zu: sx_create failed", k);
         rc = sx_stage(w.ctx, t.xyz, t.NA, t.NF, t.layout);
+        // (a batch holds many contexts, each staged once)
+        w.ctx->stage.release();
+        w.ctx->stage2.release();
         if (rc == SX_OK) rc = sx_set_factors(w.ctx, t.b, t.NA);
         if (rc != SX_OK) return bfail(b, rc, "trajectory %zu: %s", k, sx_last_error(w.ctx));
         if (!w.ctx->plan_ok || w.ctx->plan.N1 > 1)

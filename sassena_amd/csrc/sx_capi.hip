@@ -195,12 +195,24 @@ int pick_all_split(sx_ctx *c, int V, int vb, bool per_row, int *split) {
     return SX_OK;
 }
 
+// Transpose buffers up to this size are kept between blocks.
+constexpr size_t kStageKeepBytes = (size_t)16 << 20;
+
 // Largest buffer of per-pair parts of a the split "self" path may use.
 constexpr size_t kSplitBudgetBytes = (size_t)16 << 30;
 
+// The FFT plan and tables of the staged number of frames, which alone they depend
+// on: kept from one block to the next of as many frames (host sines, six
+// copies and the weights: 1,000 atoms x 200 frames staged and scanned at 10 shells x
+// 50 vectors 490 -> 374 us with this and the transpose buffer kept).
 int prepare_tables(sx_ctx *c) {
+    if (c->tables_NF == c->NF) return SX_OK;
+    c->tables_NF = 0;
     c->plan_ok = sx::make_fft_plan(c->NF, &c->plan);
-    if (!c->plan_ok) return SX_OK;  // only the autocorrelation needs it
+    if (!c->plan_ok) {  // only the autocorrelation needs it
+        c->tables_NF = c->NF;
+        return SX_OK;
+    }
     const int L = c->plan.L;
     std::vector<float2> tw(L);
     std::vector<double2> twf(L), tw64(L);
@@ -238,6 +250,7 @@ int prepare_tables(sx_ctx *c) {
     SX_HIP(c, hipMemcpyAsync(c->twp.p, tp.data(), sizeof(float2) * P.ntw, hipMemcpyHostToDevice, c->stream));
     SX_HIP(c, hipMemcpyAsync(c->twp64.p, tp64.data(), sizeof(double2) * P.ntw, hipMemcpyHostToDevice, c->stream));
     SX_HIP(c, hipStreamSynchronize(c->stream));
+    c->tables_NF = c->NF;
     return SX_OK;
 }
 
@@ -1005,7 +1018,7 @@ int stage_upload(sx_ctx *c, const float *xyz, size_t NA, size_t NF, int layout, 
     const bool aos = layout != SX_LAYOUT_SOA;
     if (aos) {
         SX_HIP(c, c->stage.ensure(sizeof(float) * maxf));
-        SX_HIP(c, c->stage2.ensure(sizeof(float) * maxf));
+        if (pieces.size() > 1) SX_HIP(c, c->stage2.ensure(sizeof(float) * maxf));
     }
     hipEvent_t done[2] = {nullptr, nullptr};
     SX_HIP(c, hipEventCreateWithFlags(&done[0], hipEventDisableTiming));
@@ -1090,8 +1103,9 @@ int sx_stage(sx_ctx *c, const float *xyz, size_t NA, size_t NF, int layout) {
     std::memcpy(&amax, &bits, sizeof amax);
     c->rmax = std::sqrt(3.0) * (double)amax;
     if (!std::isfinite(c->rmax)) return fail(c, SX_ERR_ARG, "sx_stage: non-finite coordinates");
-    c->stage.release();
-    c->stage2.release();
+    // the transpose's buffers stay for the next block while small
+    for (DevBuf *buf : {&c->stage, &c->stage2})
+        if (buf->cap > kStageKeepBytes) buf->release();
     rc = prepare_tables(c);
     if (rc != SX_OK) return rc;
     c->staged = true;

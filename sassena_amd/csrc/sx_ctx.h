@@ -86,6 +86,7 @@ struct sx_ctx {
         mpang, mptab, mpsum, qres, redbuf, pack, fparts;
     sx_timing timing{};
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
+    size_t tables_NF = 0;  // frames that the FFT plan and tables are for, 0: none
     // stepping mode of the oriented shells of the current call (sx::shell_progression:
     // 0 none, 1 exact progression, 2 progression with first-order residual corrections);
     // origin and step in |q| / 2 pi
