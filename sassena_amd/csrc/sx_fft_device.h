@@ -452,15 +452,18 @@ struct MidTwiddles {
         twp = tw;
         if constexpr (kKept) load_from<1>(tw, ut);
     }
-    // the twiddles of pass p (Ns <= T) into t
+    // the twiddles of pass p (Ns <= T): those kept, or loaded into t.  (A copy of the
+    // kept ones changes which products the compiler fuses, and FP32 spectra with them.)
     template <int p>
-    __device__ __forceinline__ void pass(C (&t)[8], unsigned ut) const {
-        constexpr int R = PT::radix(p);
-        const unsigned kk = ut & (PT::ns(p) - 1);
+    __device__ __forceinline__ const C (&pass(C (&t)[8], unsigned ut) const)[8] {
+        if constexpr (kKept) {
+            return w[p];
+        } else {
+            constexpr int R = PT::radix(p);
+            const unsigned kk = ut & (PT::ns(p) - 1);
 #pragma unroll
-        for (int q = 1; q < R; ++q) {
-            if constexpr (kKept) t[q] = w[p][q];
-            else t[q] = twiddle_load(twp, kk * R, PT::toff(p) + q);
+            for (int q = 1; q < R; ++q) t[q] = twiddle_load(twp, kk * R, PT::toff(p) + q);
+            return t;
         }
     }
 };
@@ -511,8 +514,8 @@ __device__ __forceinline__ void spass_mid(C (&v)[E], C *buf, const MidTwiddles<C
     } else {
         // every group of the thread has the twiddle index kk = ut mod Ns
         const unsigned kk = ut & (Ns - 1);
-        C ws[8];
-        mt.template pass<p>(ws, ut);
+        C wt[8];
+        const C(&ws)[8] = mt.template pass<p>(wt, ut);
         const unsigned rb = PT::swz(p - 1, ut);
 #pragma unroll
         for (int i = 0; i < E / R; ++i)
@@ -631,8 +634,8 @@ __device__ __forceinline__ void spass_last_fused(C (&v)[E], Acc (&acc)[2][E], co
     C base[RB];
 #pragma unroll
     for (int b = 1; b < RB; ++b) base[b] = twiddle_load(twp, ut * RB, PT::toff(pb) + b);
-    C wa[8];
-    mt.template pass<pa>(wa, ut);
+    C wt[8];
+    const C(&wa)[8] = mt.template pass<pa>(wt, ut);
     const unsigned rb = PT::swz(pa - 1, ut);
 #pragma unroll
     for (int q = 0; q < R; ++q) v[q] = buf[rb + q * T];
@@ -696,7 +699,15 @@ __device__ __forceinline__ void fft_sweep_fixed(C (&v)[E], Acc (&acc)[2][E], C *
                                                 const Input &in, double &ar, double &ai, unsigned ut) {
     static_assert(H == 0 || Input::kPretwiddled, "the odd-bin half needs its input pre-twiddled");
     spass_first<C, E, PT>(v, buf, in, ut);
-    fft_sweep_rest<C, E, PT, H>(v, acc, buf, tw, mt, w, ar, ai, ut);
+    // (not through fft_sweep_rest: FP32 spectra follow the compiler's choice of the
+    // products that it fuses, which the nesting changes)
+    if constexpr (fused_last<PT, E>()) {
+        spass_mids<C, E, PT, 1, PT::npass - 2>(v, buf, mt, ut);
+        spass_last_fused<C, E, PT, H>(v, acc, buf, tw, mt, w, ar, ai, ut);
+    } else {
+        spass_mids<C, E, PT, 1, PT::npass - 1>(v, buf, mt, ut);
+        spass_last<C, E, PT, H>(v, acc, buf, tw, w, ar, ai, ut);
+    }
 }
 
 // The first pass from the points v[i R + q] = x(ut + i T + q Lh / R), then the rest.
