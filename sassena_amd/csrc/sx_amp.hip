@@ -180,9 +180,12 @@ __global__ __launch_bounds__(256) void amp_all_kernel(AmpKernelArgs a) {
 
     const size_t j0 = (size_t)sp * a.atoms_per_split;
     const size_t j1 = min(a.NAp, j0 + (size_t)a.atoms_per_split);
-    const float *__restrict__ X = a.X + t;
-    const float *__restrict__ Y = a.Y + t;
-    const float *__restrict__ Z = a.Z + t;
+    // buffer loads: the batch's first row as the base, the atom's row as the scalar and
+    // the lane's frame as the vector offset, so that no VALU instruction goes on addresses
+    // (601 for 8 atoms x 8 vectors, 626 with plain loads: 2.90 -> 2.78 ms a call of 20,000
+    // atoms x 2,000 frames x 200 vectors)
+    const unsigned voff = (unsigned)(t * sizeof(float));
+    const int rows = (int)(kAtomChunk * a.NFp * sizeof(float));
 
     for (size_t jf = j0; jf < j1; jf += kFold) {
         const size_t jend = min(j1, jf + (size_t)kFold);
@@ -192,11 +195,18 @@ __global__ __launch_bounds__(256) void amp_all_kernel(AmpKernelArgs a) {
 #pragma unroll 1
         for (size_t j = jf; j < jend; j += kAtomChunk) {
             float xs[kAtomChunk], ys[kAtomChunk], zs[kAtomChunk];
+            const __amdgpu_buffer_rsrc_t rx =
+                __builtin_amdgcn_make_buffer_rsrc((void *)(a.X + j * a.NFp), (short)0, rows, kBufferDword3);
+            const __amdgpu_buffer_rsrc_t ry =
+                __builtin_amdgcn_make_buffer_rsrc((void *)(a.Y + j * a.NFp), (short)0, rows, kBufferDword3);
+            const __amdgpu_buffer_rsrc_t rz =
+                __builtin_amdgcn_make_buffer_rsrc((void *)(a.Z + j * a.NFp), (short)0, rows, kBufferDword3);
 #pragma unroll
             for (int c = 0; c < kAtomChunk; ++c) {
-                xs[c] = X[(j + c) * a.NFp];
-                ys[c] = Y[(j + c) * a.NFp];
-                zs[c] = Z[(j + c) * a.NFp];
+                const int so = (int)(c * a.NFp * sizeof(float));
+                xs[c] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rx, voff, so, 0));
+                ys[c] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(ry, voff, so, 0));
+                zs[c] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rz, voff, so, 0));
             }
 #pragma unroll
             for (int c = 0; c < kAtomChunk; ++c) {
