@@ -16,9 +16,17 @@
 // every stage is a few MFMAs deep; the weights are kept as ready operand
 // fragments (8 B a lane, loaded at the start straight into registers);
 // activations and their derivatives pass between wavefronts through LDS, as
-// fragments for the weight gradients and as rows for the next layer; the weight
-// gradients sum their 64 rows in the accumulators and leave as fragments.  A
-// second launch sums the workgroups' partials in a fixed order and applies Adam.
+// fragments for the weight gradients and as rows for the next layer.  A second
+// launch sums the workgroups' partials and applies Adam.
+//
+// Every sum has one order, whichever wavefronts hold its terms, so that results
+// neither vary from run to run nor follow the layout: an output adds its columns
+// tile after tile, then over the 16 of a tile; a workgroup's weight gradients
+// are those of its 16-row tiles added one after the other, as are db3 and the
+// loss; the gradients of its columns are those of its 4-row groups; the
+// workgroups follow in order.  Products that enter a sum do so by fmaf, which
+// leaves the compiler no choice of which one to fuse.  (Adam carries a rounding
+// of one sum into the fourth digit of the parameters within 500 steps.)
 // 4,096 rows a step: 14 + 5 us (133 + 16 us when each of four wavefronts took 16
 // rows through all columns, copied W2 into LDS and added its gradients there
 // by LDS atomics).
@@ -91,22 +99,22 @@ struct StepArgs {
 // A operand start in different banks.
 constexpr int LD = H + 4;
 
-// Sum over the four lane groups (rows of a D tile) of a per-lane column value.
-__device__ __forceinline__ float col_sum(float x) {
-    x += __shfl_xor(x, 16, 64);
-    x += __shfl_xor(x, 32, 64);
-    return x;
-}
-
 // Forward (and backward when a.t != nullptr) of ROWS_PER_BLOCK rows.
 __global__ __launch_bounds__(kStepThreads) void mlp_step_kernel(StepArgs a) {
     __shared__ short rows_lds[ROWS_PER_BLOCK * LD];  // h1, then dz2: A operands
     __shared__ bf16x4 h1f[4 * 8 * 64];               // D tiles [row tile][column tile][lane]
-    __shared__ bf16x4 dzf[4 * 8 * 64];               // dz2, then dz1
     __shared__ bf16x4 xf[4 * 64];                    // x^T: A operand of dW1
-    __shared__ float ypart[4][ROWS_PER_BLOCK];       // per column quarter
-    __shared__ float cols[3][4][H];                  // db1, db2, dW3 per row tile
-    __shared__ float sums[2][4];                     // db3 and loss per row tile
+    __shared__ float yrow[ROWS_PER_BLOCK];
+    __shared__ float sums[2][16];                    // db3 and loss per 4-row group
+    __shared__ union {
+        float h2[4][4][8][64];                       // [row tile][row mod 4][column tile][lane]
+        struct {
+            bf16x4 dzf[4 * 8 * 64];                  // dz2, then dz1: D tiles
+            float cols[3][16][H];                    // db1, db2, dW3 per 4-row group
+        };
+    } u;
+    bf16x4 *dzf = u.dzf;
+    auto &cols = u.cols;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int rt = wave & 3, cq = wave >> 2;         // row tile, column quarter (tiles 2 cq, 2 cq + 1)
     const bool train = a.t != nullptr;
@@ -184,26 +192,33 @@ __global__ __launch_bounds__(kStepThreads) void mlp_step_kernel(StepArgs a) {
             const float bias = a.p[OFF_B2 + c];
             w3[i] = a.p[OFF_W3 + c];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) h2[i][j] = tanhf(acc[i][j] + bias);
+            for (int j = 0; j < 4; ++j) {
+                h2[i][j] = tanhf(acc[i][j] + bias);
+                u.h2[rt][j][2 * cq + i][lane] = h2[i][j];
+            }
         }
     }
-    // ---- layer 3: y[r] = h2[r] . W3 + b3, over the 16 lanes of a k group and the four quarters
+    __syncthreads();
+    // ---- layer 3: y[r] = h2[r] . W3 + b3, rows 4 lg + cq: tile after tile, then
+    // over the 16 lanes of a k group
+    {
+        float s = 0.f;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        float s = h2[0][j] * w3[0] + h2[1][j] * w3[1];
+        for (int nt = 0; nt < 8; ++nt) s = fmaf(u.h2[rt][cq][nt][lane], a.p[OFF_W3 + 16 * nt + lr], s);
 #pragma unroll
         for (int off = 8; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-        if (lr == 0) ypart[cq][rt * 16 + 4 * lg + j] = s;
-    }
-    __syncthreads();
-    float yr[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int r = rt * 16 + 4 * lg + j;
-        yr[j] = ((ypart[0][r] + ypart[1][r]) + (ypart[2][r] + ypart[3][r])) + a.p[OFF_B3];
-        if (a.y && cq == 0 && lr == 0 && row0 + 4 * lg + j < a.rows) a.y[row0 + 4 * lg + j] = yr[j];
+        s += a.p[OFF_B3];
+        const unsigned r = 4 * lg + cq;
+        if (lr == 0) {
+            yrow[rt * 16 + r] = s;
+            if (a.y && row0 + r < a.rows) a.y[row0 + r] = s;
+        }
     }
     if (!train) return;
+    __syncthreads();  // h2 is read: dz2 and the columns' sums take its place
+    float yr[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) yr[j] = yrow[rt * 16 + 4 * lg + j];
 
     // ---- loss and dy = 2 (y - t) / rows (rows beyond the batch contribute 0)
     float dy[4], dsum = 0.f, lsum = 0.f;
@@ -212,13 +227,11 @@ __global__ __launch_bounds__(kStepThreads) void mlp_step_kernel(StepArgs a) {
         const float e = rd[j] >= 0 ? yr[j] - tv[j] : 0.f;
         dy[j] = 2.f * e / (float)a.rows;
         dsum += dy[j];
-        lsum += e * e;
+        lsum = fmaf(e, e, lsum);
     }
-    dsum = col_sum(dsum);
-    lsum = col_sum(lsum);
-    if (cq == 0 && lane == 0) {
-        sums[0][rt] = dsum;
-        sums[1][rt] = lsum;
+    if (cq == 0 && lr == 0) {
+        sums[0][rt * 4 + lg] = dsum;
+        sums[1][rt * 4 + lg] = lsum;
     }
     // ---- dz2 = dy W3 (1 - h2^2); dW3 = sum dy h2; db2 = sum dz2
 #pragma unroll
@@ -228,32 +241,29 @@ __global__ __launch_bounds__(kStepThreads) void mlp_step_kernel(StepArgs a) {
         bf16x4 f;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const float dz = dy[j] * w3[i] * (1.f - h2[i][j] * h2[i][j]);
-            gw3 += dy[j] * h2[i][j];
-            gb2 += dz;
-            f[j] = to_bf16(dz);
+            const float dw = dy[j] * w3[i], d = fmaf(-h2[i][j], h2[i][j], 1.f);
+            gw3 = fmaf(dy[j], h2[i][j], gw3);
+            gb2 = fmaf(dw, d, gb2);
+            f[j] = to_bf16(dw * d);
             rows_lds[(rt * 16 + 4 * lg + j) * LD + c] = f[j];  // h1's rows were read before the last barrier
         }
         dzf[(rt * 8 + nt) * 64 + lane] = f;
-        gw3 = col_sum(gw3);
-        gb2 = col_sum(gb2);
-        if (lg == 0) {
-            cols[2][rt][c] = gw3;
-            cols[1][rt][c] = gb2;
-        }
+        cols[2][rt * 4 + lg][c] = gw3;
+        cols[1][rt * 4 + lg][c] = gb2;
     }
     __syncthreads();
     float *dst = a.partial + (size_t)blockIdx.x * PK;
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     // ---- dW2[k][c] = sum_r h1[r][k] dz2[r][c]: A = h1^T (D tiles of h1), B = dz2 (D tiles);
-    // row of tiles wave / 2, four of its tiles
+    // row of tiles wave / 2, four of its tiles, each row tile's product added to the last
     {
         const int mt = wave >> 1, c0 = (wave & 1) * 4;
-        f32x4 acc[4] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+        f32x4 acc[4] = {zero, zero, zero, zero};
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const bf16x4 av = h1f[(r * 8 + mt) * 64 + lane];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) acc[i] = mfma(av, dzf[(r * 8 + c0 + i) * 64 + lane], acc[i]);
+            for (int i = 0; i < 4; ++i) acc[i] += mfma(av, dzf[(r * 8 + c0 + i) * 64 + lane], zero);
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i)
@@ -274,12 +284,11 @@ __global__ __launch_bounds__(kStepThreads) void mlp_step_kernel(StepArgs a) {
             float gb1 = 0.f;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const float dz = acc[i][j] * (1.f - h1[i][j] * h1[i][j]);
-                gb1 += dz;
-                d1[i][j] = to_bf16(dz);
+                const float d = fmaf(-h1[i][j], h1[i][j], 1.f);
+                gb1 = fmaf(acc[i][j], d, gb1);
+                d1[i][j] = to_bf16(acc[i][j] * d);
             }
-            gb1 = col_sum(gb1);
-            if (lg == 0) cols[0][rt][16 * (2 * cq + i) + lr] = gb1;
+            cols[0][rt * 4 + lg][16 * (2 * cq + i) + lr] = gb1;
         }
     }
     __syncthreads();  // dz2's fragments are read
@@ -288,18 +297,24 @@ __global__ __launch_bounds__(kStepThreads) void mlp_step_kernel(StepArgs a) {
     __syncthreads();
     // ---- dW1[k][c] = sum_r x[r][k] dz1[r][c]
     if (wave < 8) {
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        f32x4 acc = zero;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) acc = mfma(xf[r * 64 + lane], dzf[(r * 8 + wave) * 64 + lane], acc);
+        for (int r = 0; r < 4; ++r) acc += mfma(xf[r * 64 + lane], dzf[(r * 8 + wave) * 64 + lane], zero);
         *reinterpret_cast<f32x4 *>(dst + PK_W1 + (wave * 64 + lane) * 4) = acc;
     } else {
         const int i = tid - 512;
         if (i < 3 * H) {
-            const int q = i / H, c = i % H;
-            dst[PK_B1 + i] = (cols[q][0][c] + cols[q][1][c]) + (cols[q][2][c] + cols[q][3][c]);
+            float s = 0.f;
+#pragma unroll
+            for (int k = 0; k < 16; ++k) s += cols[i / H][k][i % H];
+            dst[PK_B1 + i] = s;
         } else if (i < 3 * H + 2) {
-            const int q = i - 3 * H;
-            dst[PK_B3 + q] = (sums[q][0] + sums[q][1]) + (sums[q][2] + sums[q][3]);
+            float s = 0.f;
+            for (int r = 0; r < 16; r += 4) {
+                const float *g = sums[i - 3 * H] + r;
+                s += ((g[0] + g[1]) + g[2]) + g[3];
+            }
+            dst[PK_B3 + i - 3 * H] = s;
         }
     }
 }
@@ -329,31 +344,42 @@ __device__ __forceinline__ void put_fragment(short *frag, int i, float v) {
     }
 }
 
-// Sums the workgroups' gradients (fixed order) into grad, and optionally
+// Sums the workgroups' gradients in their order into grad, and optionally
 // applies one Adam step to the FP32 parameters and refreshes the BF16
-// fragments.  A thread takes 4 entries of every kSlices-th workgroup; the
-// slices meet in LDS.
-constexpr int kSlices = 16, kGroups = 16;
+// fragments.  A thread loads 4 entries of every kSlices-th workgroup into LDS,
+// kStaged workgroups at a time; then each entry has a thread that adds them.
+constexpr int kSlices = 16, kGroups = 16, kStaged = 64;
 __global__ __launch_bounds__(kSlices *kGroups) void mlp_reduce_adam_kernel(
     const float *__restrict__ partial, int blocks, float *__restrict__ grad, float *__restrict__ loss,
     float *__restrict__ p, float *__restrict__ m, float *__restrict__ v, short *__restrict__ frag, int apply, float lr,
     float b1c, float b2c) {
-    __shared__ f32x4 sh[kSlices][kGroups];
+    __shared__ f32x4 sh[kStaged][kGroups];
     const int g = threadIdx.x % kGroups, sl = threadIdx.x / kGroups;
     const int e0 = ((int)blockIdx.x * kGroups + g) * 4;
-    f32x4 s = {0.f, 0.f, 0.f, 0.f};
-    if (e0 < PK) {
-#pragma unroll 4
-        for (int b = sl; b < blocks; b += kSlices) s += *reinterpret_cast<const f32x4 *>(partial + (size_t)b * PK + e0);
-    }
-    sh[sl][g] = s;
-    __syncthreads();
-    if (threadIdx.x >= kGroups * 4) return;
-    // one entry a thread
     const int gi = threadIdx.x >> 2, j = threadIdx.x & 3, e = ((int)blockIdx.x * kGroups + gi) * 4 + j;
     float gr = 0.f;
-    for (int k = 0; k < kSlices; ++k) gr += sh[k][gi][j];
-    if (e > PK_LOSS) return;
+    for (int b0 = 0; b0 < blocks; b0 += kStaged) {
+        const int nb = min(kStaged, blocks - b0);
+        f32x4 x[kStaged / kSlices];
+#pragma unroll
+        for (int k = 0; k < kStaged / kSlices; ++k) {
+            const int b = sl + k * kSlices;
+            if (b < nb && e0 < PK) x[k] = *reinterpret_cast<const f32x4 *>(partial + (size_t)(b0 + b) * PK + e0);
+        }
+#pragma unroll
+        for (int k = 0; k < kStaged / kSlices; ++k) {
+            const int b = sl + k * kSlices;
+            if (b < nb && e0 < PK) sh[b][g] = x[k];
+        }
+        __syncthreads();
+        if (threadIdx.x < kGroups * 4) {
+            // one entry a thread
+#pragma unroll 16
+            for (int b = 0; b < nb; ++b) gr += sh[b][gi][j];
+        }
+        __syncthreads();
+    }
+    if (threadIdx.x >= kGroups * 4 || e > PK_LOSS) return;
     if (e == PK_LOSS) {
         if (loss) *loss = gr;
         return;
