@@ -430,13 +430,17 @@ int mfail(sx_mlp *n, int code, const char *fmt, ...) {
 #define SXM_HIP(n, expr)                                                                                    \
     do {                                                                                                    \
         hipError_t e_ = (expr);                                                                             \
-        if (e_ != hipSuccess)                                                                               \
+        if (e_ != hipSuccess) {                                                                             \
+            (void)hipGetLastError(); /* reported here, and not by the next call's launches too */           \
             return mfail((n), e_ == hipErrorOutOfMemory ? SX_ERR_NOMEM : SX_ERR_HIP, "%s failed: %s (%s:%d)", \
                          #expr, hipGetErrorString(e_), __FILE__, __LINE__);                                 \
+        }                                                                                                   \
     } while (0)
 
+// The capacities hold only for buffers that are there: 0 until every allocation succeeded.
 int ensure_rows(sx_mlp *n, size_t rows) {
     if (rows <= n->xcap) return SX_OK;
+    n->xcap = 0;
     for (float **q : {&n->x, &n->t, &n->y})
         if (*q) {
             (void)hipFree(*q);
@@ -451,6 +455,7 @@ int ensure_rows(sx_mlp *n, size_t rows) {
 
 int ensure_partials(sx_mlp *n, size_t blocks) {
     if (blocks <= n->pcap_blocks) return SX_OK;
+    n->pcap_blocks = 0;
     if (n->partial) (void)hipFree(n->partial);
     n->partial = nullptr;
     SXM_HIP(n, hipMalloc(&n->partial, sizeof(float) * sxm::PK * blocks));
