@@ -315,13 +315,16 @@ size_t cylinder_parts_bytes(int N1, size_t NFp, int ns, int split, int sub) {
     return sizeof(double2) * 2 * N1 * NFp * (size_t)ns * split * sub;
 }
 
-// Ranges are cut into parts, of at least 32 atoms, until the wavefronts fill
-// whole rounds of the two a SIMD that fit.
+// Ranges are cut into parts, of at least 8 atoms, until the wavefronts fill
+// whole rounds of the two a SIMD that fit.  (An atom's chain of recurrences takes
+// 2 to 6 us and calls of few atoms leave SIMDs idle: 1,000 atoms x 100 frames x 1
+// shell, whole calls with parts of 32 and of 8 atoms: (16, 0) alone 319 and 179 us,
+// l <= 10 250 and 170 us.)
 int cylinder_parts_per_range(int N1, size_t NFp, size_t NAp, int ns, int split, int cus) {
     int groups = 1;
     (void)cylinder_kernel(N1, &groups);
     const long base = (long)(NFp / kWave) * ns * groups * split, resident = 8L * cus;
-    const long most = std::max<long>(1, std::min<long>(32, (long)(NAp / split / 32)));
+    const long most = std::max<long>(1, std::min<long>(32, (long)(NAp / split / 8)));
     int sub = 1;
     double best = 0.0;
     for (long s = 1; s <= most; ++s) {
