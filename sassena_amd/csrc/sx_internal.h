@@ -320,7 +320,7 @@ constexpr int kSphereSumL1 = 17;
 // What a wavefront does for one degree l of two orders m, m + 1 (m even).
 struct SphereEntry {
     double alpha1, alpha2;  // recurrence coefficients of the two orders at l
-    int l;
+    int l;                  // above the lowest degree, as f1 and f2 above the lowest order
     int skip;               // steps from degree m to l without sums, or -1: l follows the entry before
     int first;              // alpha[m][m]
     int f1, f2;             // powers of u of the two orders
@@ -328,8 +328,10 @@ struct SphereEntry {
 };
 struct SpherePlan {
     int L1 = 0, M1 = 0;        // degrees, orders
+    int l0 = 0, m0 = 0;        // the lowest of each that have entries
     int nd = 0;                // (pair of orders, degree) entries
     int kernel = -1, groups = 0, CA = 0;
+    int per_cu = 1;            // workgroups a CU that ranges are cut for
     std::vector<SphereEntry> sched;  // per wavefront, its entries
     std::vector<double> alpha; // [M1 + 1][L1] coefficients of the recurrence in the degree
     std::vector<double> scale; // [nmo] normalisation of the finished sums

@@ -37,19 +37,22 @@ namespace {
 
 constexpr int kWaves = 8;
 constexpr int kThreads = kWaves * kWave;
+constexpr int kFewEntries = 2;  // entries a wavefront of the kernels that take lists of few pairs
 constexpr double kPi = 3.14159265358979323846;
 
-// w j_l(x), l < L1, to J[l * stride]: upward where x exceeds the largest
+// w j_l(x), l0 <= l < L1, to J[l * stride]: upward where x exceeds the largest
 // degree, else by Miller's downward recurrence, normalised to j_0 or j_1; below 1e-8
 // by the leading term, x^l / (2l + 1)!!, whose relative error is x^2.
 // From 1e-8 the recurrence stays in range from its start at 1e-280.
 // Miller's recurrence starts at degree `start`.
-__device__ __forceinline__ void bessel_to_lds(double w, double x, int L1, int start, double *J, int stride) {
+// (LOW: l0 may be above 0; without it the loops stay those of all degrees.)
+template <bool LOW>
+__device__ __forceinline__ void bessel_to_lds(double w, double x, int l0, int L1, int start, double *J, int stride) {
     if (x < 1e-8) {
         double j = w;
 #pragma unroll 1
         for (int l = 0; l < L1; ++l) {
-            J[l * stride] = j;
+            if (!LOW || l >= l0) J[l * stride] = j;
             j *= x / (2.0 * l + 3.0);
         }
         return;
@@ -60,11 +63,18 @@ __device__ __forceinline__ void bessel_to_lds(double w, double x, int L1, int st
     const double j0 = w * s * ix, j1 = fma(-w, c, j0) * ix;
     const int L = L1 - 1;
     if (x > (double)L) {
-        J[0] = j0;
-        if (L1 > 1) J[stride] = j1;
+        if (!LOW || l0 == 0) J[0] = j0;
+        if (L1 > 1 && (!LOW || l0 <= 1)) J[stride] = j1;
         double a = j0, b = j1;
+        int l = 2;
+#pragma unroll 1
+        for (; LOW && l < l0; ++l) {
+            const double n = fma((2.0 * l - 1.0) * ix, b, -a);
+            a = b;
+            b = n;
+        }
 #pragma unroll 2
-        for (int l = 2; l < L1; ++l) {
+        for (; l < L1; ++l) {
             const double n = fma((2.0 * l - 1.0) * ix, b, -a);
             a = b;
             b = n;
@@ -80,19 +90,26 @@ __device__ __forceinline__ void bessel_to_lds(double w, double x, int L1, int st
         fp1 = f;
         f = fm1;
     }
+    const int low = LOW ? max(l0, 2) : 1;
 #pragma unroll 2
-    for (; n > 0; --n) {
+    for (; n >= low; --n) {
         J[n * stride] = f;
+        const double fm1 = fma((2.0 * n + 1.0) * ix, f, -fp1);
+        fp1 = f;
+        f = fm1;
+    }
+#pragma unroll 1
+    for (; LOW && n > 0; --n) {
         const double fm1 = fma((2.0 * n + 1.0) * ix, f, -fp1);
         fp1 = f;
         f = fm1;
     }
     // f = f_0, fp1 = f_1
     const double sc = fabs(j0) >= fabs(j1) || L == 0 ? j0 / f : j1 / fp1;
-    J[0] = j0;
-    if (L >= 1) J[stride] = j1;
+    if (!LOW || l0 == 0) J[0] = j0;
+    if (L >= 1 && (!LOW || l0 <= 1)) J[stride] = j1;
 #pragma unroll 1
-    for (int l = 2; l < L1; ++l) J[l * stride] *= sc;
+    for (int l = LOW ? low : 2; l < L1; ++l) J[l * stride] *= sc;
 }
 
 struct SphereSumArgs {
@@ -103,6 +120,7 @@ struct SphereSumArgs {
     int per_shell_b;
     const double *q;                        // |q| per shell
     int ns, L1, M1, CA, sub;                // degrees, orders, atoms per step, parts per range
+    int l0, m0;                             // lists of few pairs: the lowest degree and order that have entries
     int start;                              // of Miller's recurrence, L + 32 + 2 sqrt(2 L) for x <= L
     int nd;                                 // pairs of orders x degree in all
     const SphereEntry *sched;               // [kWaves][ND]
@@ -120,8 +138,12 @@ __global__ __launch_bounds__(kThreads) void sphere_sums_kernel(SphereSumArgs a) 
     const size_t r0 = (size_t)(z / a.sub) * a.range, r1 = min(a.NAp, r0 + a.range);
     const size_t len = r1 > r0 ? r1 - r0 : 0;
     const size_t j0 = r0 + len * (z % a.sub) / a.sub, j1 = r0 + len * (z % a.sub + 1) / a.sub;
-    // LDS of one atom: J [L1][MS][64], F [M1] double2 [64], cos theta [64]
-    const int per_atom = (a.L1 * MS + 2 * a.M1 + 1) * kWave;
+    // LDS of one atom, from the lowest degree and order on: J [L1 - l0][MS][64],
+    // F [M1 - m0] double2 [64], cos theta [64]
+    constexpr bool LOW = ND == kFewEntries;
+    const int l0 = LOW ? a.l0 : 0, m0 = LOW ? a.m0 : 0;
+    const int jrows = (a.L1 - l0) * MS, frows = 2 * (a.M1 - m0);
+    const int per_atom = (jrows + frows + 1) * kWave;
 
     const auto alpha = uniform(a.alpha), Q = uniform(a.q);
     const auto B = uniform(a.b);
@@ -147,30 +169,31 @@ __global__ __launch_bounds__(kThreads) void sphere_sums_kernel(SphereSumArgs a) 
                 const int sh = min(s0 + s, a.ns - 1);
                 const float w = B[(a.per_shell_b ? (size_t)sh * a.NAp : 0) + j];
                 if (w == 0.f) {
-                    for (int l = 0; l < a.L1; ++l) J[l * (MS * kWave)] = 0.0;
+                    for (int l = 0; l < a.L1 - l0; ++l) J[l * (MS * kWave)] = 0.0;
                 } else {
-                    bessel_to_lds((double)w, Q[sh] * (double)a.srf[e], a.L1, a.start, J, MS * kWave);
+                    bessel_to_lds<LOW>((double)w, Q[sh] * (double)a.srf[e], l0, a.L1, a.start, J - l0 * (MS * kWave),
+                                       MS * kWave);
                 }
             } else {
                 const double st = a.sst[e], ur = -st * a.scp[e], ui = -st * a.ssp[e];
-                double2 *F = reinterpret_cast<double2 *>(lds + c * per_atom + a.L1 * MS * kWave) + lane;
+                double2 *F = reinterpret_cast<double2 *>(lds + c * per_atom + jrows * kWave) + lane;
                 double fr = 1.0, fi = 0.0;
 #pragma unroll 1
                 for (int m = 0; m < a.M1; ++m) {
-                    F[m * kWave] = make_double2(fr, fi);
+                    if (!LOW || m >= m0) F[(m - m0) * kWave] = make_double2(fr, fi);
                     const double nr = fma(fr, ur, -fi * ui);
                     fi = fma(fr, ui, fi * ur);
                     fr = nr;
                 }
-                A[(a.L1 * MS + 2 * a.M1) * kWave] = a.sct[e];
+                A[(jrows + frows) * kWave] = a.sct[e];
             }
         }
         __syncthreads();
 #pragma unroll 1
         for (int c = 0; c < na; ++c) {
             const double *A = lds + c * per_atom + lane;
-            const double2 *F = reinterpret_cast<const double2 *>(lds + c * per_atom + a.L1 * MS * kWave) + lane;
-            const double ct = A[(a.L1 * MS + 2 * a.M1) * kWave];
+            const double2 *F = reinterpret_cast<const double2 *>(lds + c * per_atom + jrows * kWave) + lane;
+            const double ct = A[(jrows + frows) * kWave];
             double ta1 = 0.0, tb1 = 0.0, ta2 = 0.0, tb2 = 0.0;
             double2 f1 = make_double2(0.0, 0.0), f2 = f1;
             // the wavefront's entries, read again for every atom through an index
@@ -283,8 +306,18 @@ const SumsKernel kKernels[] = {
     {11, 1, sphere_sums_kernel<1, 11>}, {11, 2, sphere_sums_kernel<2, 11>},
 };
 constexpr size_t kLdsBytes = 160 << 10;
+// Lists of at most one pair a wavefront: the sums no longer cover the latency of
+// the factors' loads and chains, so that workgroups take at most 3 shells and half
+// of the LDS, which then starts at their lowest degree and order, so that two and
+// more share a CU, and ranges are cut for four.  5,000 atoms x 2,000 frames x 5 shells,
+// whole calls: (0, 0) 1.72 -> 1.17 ms, l <= 3 1.98 -> 1.43 ms, (16, 0) 3.43 -> 2.86 ms,
+// (16, 16) 3.20 -> 2.46 ms (2.76 ms by the moment's own recurrence from a table of
+// Bessel functions; the other single moments were no faster that way either).
+constexpr int kFewShells = 3, kFewPerCu = 4;
 
-size_t lds_per_atom(int L1, int ms, int M1) { return sizeof(double) * kWave * ((size_t)L1 * ms + 2 * M1 + 1); }
+size_t lds_per_atom(int degrees, int ms, int orders) {
+    return sizeof(double) * kWave * ((size_t)degrees * ms + 2 * orders + 1);
+}
 
 }  // namespace
 
@@ -310,13 +343,22 @@ bool make_sphere_plan(const int *moments, int nmo, int ns, SpherePlan *plan) {
             }
     p.nd = (int)pairs.size();
     const int per_wave = (p.nd + kWaves - 1) / kWaves;
+    const bool few = per_wave == 1;
+    if (few) {
+        p.l0 = pairs[0].x;
+        for (const int2 &q : pairs) p.l0 = std::min(p.l0, q.x);
+        p.m0 = pairs[0].y;
+    }
+    const int degrees = p.L1 - p.l0, orders = p.M1 - p.m0;
+    p.per_cu = few ? kFewPerCu : 1;
     // the kernel of the fewest operations: 8 a pair and 4 a pair and shell,
     // about 80 a shell for its Bessel functions, 60 for the angles, per group of shells
     double best = 0.0;
     p.kernel = -1;
     for (int i = 0; i < (int)(sizeof(kKernels) / sizeof(kKernels[0])); ++i) {
         const SumsKernel &k = kKernels[i];
-        if (k.nd < per_wave || lds_per_atom(p.L1, k.ms, p.M1) > kLdsBytes) continue;
+        if (few && (k.nd != kFewEntries || k.ms > kFewShells)) continue;
+        if (k.nd < per_wave || lds_per_atom(degrees, k.ms, orders) > kLdsBytes) continue;
         const int groups = (ns + k.ms - 1) / k.ms;
         const double cost = groups * (p.nd * (8.0 + 4.0 * k.ms) + 80.0 * k.ms + 60.0) + 0.01 * k.nd;
         if (p.kernel < 0 || cost < best) {
@@ -327,7 +369,7 @@ bool make_sphere_plan(const int *moments, int nmo, int ns, SpherePlan *plan) {
     if (p.kernel < 0) return false;
     const SumsKernel &kk = kKernels[p.kernel];
     p.groups = (ns + kk.ms - 1) / kk.ms;
-    p.CA = (int)std::min<size_t>(8, kLdsBytes / lds_per_atom(p.L1, kk.ms, p.M1));
+    p.CA = (int)std::max<size_t>(1, std::min<size_t>(8, kLdsBytes / (few ? 2 : 1) / lds_per_atom(degrees, kk.ms, orders)));
     // P_lm normalised as Y_lm: P_l = a_l (x P_{l-1} - e_l P_{l-2}), a_l =
     // sqrt((4 l^2 - 1) / (l^2 - m^2)), e_l = sqrt(((l-1)^2 - m^2) / (4 (l-1)^2 - 1));
     // P_l = s_l T_l with s_l = a_l e_l s_{l-2}
@@ -356,11 +398,11 @@ bool make_sphere_plan(const int *moments, int nmo, int ns, SpherePlan *plan) {
             SphereEntry &e = p.sched[(size_t)w * kk.nd + d - d0];
             e.alpha1 = p.alpha[(size_t)m * p.L1 + l];
             e.alpha2 = p.alpha[(size_t)(m + 1) * p.L1 + l];
-            e.l = l;
+            e.l = l - p.l0;
             e.skip = next ? -1 : l - m;
             e.first = m * p.L1 + m;
-            e.f1 = m;
-            e.f2 = std::min(m + 1, mmax);
+            e.f1 = m - p.m0;
+            e.f2 = std::min(m + 1, mmax) - p.m0;
             e.pair = d;
         }
     }
@@ -380,15 +422,16 @@ size_t sphere_parts_bytes(const SpherePlan &p, size_t NFp, int ns, int split, in
     return sizeof(double2) * 2 * p.nd * NFp * (size_t)ns * split * sub;
 }
 
-// One workgroup a CU (LDS and registers): ranges are cut into parts, of at
-// least 32 atoms, until the workgroups fill whole rounds of the CUs.
+// One workgroup a CU (LDS and registers; per_cu for lists of few pairs): ranges
+// are cut into parts, of at least 32 atoms, until the workgroups fill whole
+// rounds of the CUs.
 int sphere_parts_per_range(const SpherePlan &p, size_t NFp, size_t NAp, int split, int cus) {
-    const long base = (long)(NFp / kWave) * p.groups * split;
+    const long base = (long)(NFp / kWave) * p.groups * split, resident = (long)cus * p.per_cu;
     const long most = std::max<long>(1, std::min<long>(32, (long)(NAp / split / 32)));
     int sub = 1;
     double best = 0.0;
     for (long s = 1; s <= most; ++s) {
-        const double rounds = (double)((base * s + cus - 1) / cus) / (double)s;
+        const double rounds = (double)((base * s + resident - 1) / resident) / (double)s;
         if (s == 1 || rounds < best * 0.97) {
             best = rounds;
             sub = (int)s;
@@ -436,6 +479,8 @@ hipError_t launch_sphere_sums(const MultipoleArgs &m, const SpherePlan &p, const
     a.M1 = p.M1;
     a.CA = p.CA;
     a.sub = sub;
+    a.l0 = p.l0;
+    a.m0 = p.m0;
     a.start = p.L1 - 1 + 32 + (int)(2.0 * std::sqrt(2.0 * (p.L1 - 1)));
     a.nd = p.nd;
     const char *tb = static_cast<const char *>(tables);
@@ -445,7 +490,7 @@ hipError_t launch_sphere_sums(const MultipoleArgs &m, const SpherePlan &p, const
     const int2 *entry = reinterpret_cast<const int2 *>(scale + p.scale.size());
     a.parts = static_cast<double2 *>(parts);
     const SumsKernel &k = kKernels[p.kernel];
-    const size_t lds = lds_per_atom(p.L1, k.ms, p.M1) * p.CA;
+    const size_t lds = lds_per_atom(p.L1 - p.l0, k.ms, p.M1 - p.m0) * p.CA;
     hipError_t e =
         hipFuncSetAttribute((const void *)k.fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;

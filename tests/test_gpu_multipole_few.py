@@ -1,4 +1,6 @@
-"""Multipole calls of few atoms, cylinder ranges cut into parts of eight atoms, against the kernel that runs every
+"""Multipole lists of few moments and calls of few atoms: sphere lists of at most
+eight pairs of orders, whose factors start at their lowest degree and order, and
+cylinder ranges cut into parts of eight atoms, against the kernel that runs every
 recurrence per moment (multipole_terms = 3): the same atom ranges in FP64, so
 amplitudes differ by at most one FP32 rounding, 2^-23 relative in F."""
 import numpy as np
@@ -33,6 +35,14 @@ def compare(kind, moments, ns, NA, NF, split, axis=(0.0, 0.0, 1.0)):
     assert np.max(np.abs(a[0] - r[0]) / f0) < TOL
     assert np.max(np.abs(a[1] - r[1]) / f0[:, 0]) < TOL
     assert np.max(np.abs(a[2] - r[2]) / f0[:, 0] ** 2) < 2 * TOL * a[0].shape[1]
+
+
+@pytest.mark.parametrize("moments", [[(0, 0)], [(1, 0)], [(1, -1)], [(2, 2), (2, -2)], [(16, 0)], [(16, -16)], [(15, 15), (16, 15)],
+                                     [(3, 2), (5, 3), (4, -2)], [(12, 5), (0, 0)], [(l, 8) for l in range(9, 17)],
+                                     [(l, m) for l in range(4) for m in range(-l, l + 1)]])
+@pytest.mark.parametrize("ns,NA,NF,split", [(1, 1, 1, 1), (3, 33, 64, 1), (4, 300, 70, 2)])
+def test_sphere_lists_of_few_pairs(moments, ns, NA, NF, split):
+    compare("sphere", moments, ns, NA, NF, split)
 
 
 @pytest.mark.parametrize("moments", [[(0, 0)], [(1, 2)], [(16, 0)], [(10, 1), (11, 3)], [(8, 2), (0, 0), (1, 1)],
