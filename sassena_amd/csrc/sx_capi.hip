@@ -130,8 +130,9 @@ int pick_split(const sx_ctx *c, int V, int vb) {
 constexpr size_t kSplitAmpBudget = (size_t)4 << 30;
 // Largest buffer of per-(atom, frame) spherical terms of the sphere multipole path.
 constexpr size_t kSphereTermBudget = (size_t)16 << 30;
-// The partial sums of a multipole call: at most this much, and only while
-// this much device memory stays free beside them.
+// The work memory of a multipole call's sums (partial sums, and the cylinder's
+// angles): at most this much, and only while this much device memory stays free
+// beside it.
 constexpr size_t kMultipoleSumBudget = (size_t)96 << 30;
 constexpr size_t kMultipoleSumMargin = (size_t)4 << 30;
 
@@ -596,12 +597,12 @@ int run_batch(sx_ctx *c, int ns, size_t NM, const double *qv, const double *qlen
                     return mp->kind == 0 ? sx::sphere_parts_bytes(sp, c->NFp, ns, split, parts)
                                          : sx::cylinder_parts_bytes(N1, c->NFp, ns, split, parts);
                 };
-                while (sub > 0 && !multipole_buffer_fits(c->mpsum, part_bytes(sub))) sub /= 2;
+                // (one buffer: parts, then the cylinder's angles)
                 const size_t angle_bytes = mp->kind == 1 ? sizeof(double2) * c->NAp * c->NFp : 0;
-                if (sub > 0 && angle_bytes > 0 && !multipole_buffer_fits(c->mpang, angle_bytes + part_bytes(sub))) sub = 0;
+                while (sub > 0 && !multipole_buffer_fits(c->mpsum, part_bytes(sub) + angle_bytes)) sub /= 2;
                 const size_t j01_bytes = sizeof(double2) * (size_t)ns * c->NAp * c->NFp;
                 if (sub > 0) {
-                    SX_HIP(c, c->mpsum.ensure(part_bytes(sub)));
+                    SX_HIP(c, c->mpsum.ensure(part_bytes(sub) + angle_bytes));
                     if (mp->kind == 0) {
                         std::vector<char> tables(sx::sphere_table_bytes(sp));
                         sx::sphere_tables(sp, tables.data());
@@ -610,8 +611,8 @@ int run_batch(sx_ctx *c, int ns, size_t NM, const double *qv, const double *qlen
                                                  c->stream));
                         SX_HIP(c, sx::launch_sphere_sums(ma, sp, c->mptab.p, sub, c->mpsum.p, c->stream));
                     } else {
-                        SX_HIP(c, c->mpang.ensure(angle_bytes));
-                        SX_HIP(c, sx::launch_cylinder_sums(ma, N1, sub, c->mpang.p, c->mpsum.p, c->stream));
+                        void *angles = static_cast<char *>(c->mpsum.p) + part_bytes(sub);
+                        SX_HIP(c, sx::launch_cylinder_sums(ma, N1, sub, angles, c->mpsum.p, c->stream));
                     }
                     summed = true;
                 } else if (j01_bytes <= kSphereTermBudget) {
@@ -926,7 +927,7 @@ void sx_destroy(sx_ctx *c) {
     if (!c) return;
     (void)hipSetDevice(c->cfg.device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
-    for (DevBuf *d : {&c->coords, &c->b, &c->twL, &c->twL64, &c->twp, &c->twp64, &c->tw64, &c->w, &c->aidx, &c->apair, &c->tail, &c->qrev, &c->qlen, &c->uvec, &c->brow, &c->bshell, &c->mpmom, &c->mpq, &c->mpsph, &c->mpj, &c->mpang, &c->mptab, &c->mpsum, &c->qres, &c->redbuf, &c->pack, &c->fparts, &c->amp,
+    for (DevBuf *d : {&c->coords, &c->b, &c->twL, &c->twL64, &c->twp, &c->twp64, &c->tw64, &c->w, &c->aidx, &c->apair, &c->tail, &c->qrev, &c->qlen, &c->uvec, &c->brow, &c->bshell, &c->mpmom, &c->mpq, &c->mpsph, &c->mpj, &c->mptab, &c->mpsum, &c->qres, &c->redbuf, &c->pack, &c->fparts, &c->amp,
                       &c->ppart, &c->apart, &c->fqt, &c->fq, &c->fq2, &c->stage, &c->stage2})
         d->release();
     for (auto &e : c->ev)

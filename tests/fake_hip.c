@@ -130,8 +130,8 @@ int hipMemcpyAsync(void *d, const void *s, size_t n, int k, void *st) { (void)k,
 int hipMemcpy(void *d, const void *s, size_t n, int k) { (void)k; drain(); memcpy(d, s, n); return kOk; }
 int hipMemcpy2DAsync(void *d, size_t dp, const void *s, size_t sp, size_t w, size_t h, int k, void *st) {
     (void)k, (void)st;
-    for (size_t i = 0; i < h; ++i)
-        if (push((char *)d + i * dp, (const char *)s + i * sp, w, 0, 0)) return kInvalid;
+    drain();
+    for (size_t i = 0; i < h; ++i) memcpy((char *)d + i * dp, (const char *)s + i * sp, w);
     return kOk;
 }
 int hipMemsetAsync(void *d, int v, size_t n, void *s) { (void)s; return push(d, NULL, n, 1, v); }
