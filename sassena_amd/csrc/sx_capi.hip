@@ -156,14 +156,22 @@ int round_filling_split(long base, int first, long resident, size_t NAp, size_t 
     return split;
 }
 
-// Whether `buf` may hold `bytes`: within the budget, and with
-// kMultipoleSumMargin of device memory left beside it.
-bool multipole_buffer_fits(const DevBuf &buf, size_t bytes) {
-    if (bytes > kMultipoleSumBudget) return false;
+// The packed atoms and FP64 parts of a call of few frames: at most as much as
+// the amplitudes, and only while this much device memory stays free beside them
+// (the correlation of so few frames takes some megabytes).
+constexpr size_t kFewMargin = (size_t)256 << 20;
+
+// Whether `buf` may hold `bytes`: with `margin` of device memory left beside
+// it, unless it does already.
+bool buffer_fits(const DevBuf &buf, size_t bytes, size_t margin) {
     if (buf.p && bytes <= buf.cap) return true;
     size_t fr = 0, tot = 0;
     if (hipMemGetInfo(&fr, &tot) != hipSuccess) return false;
-    return fr + buf.cap >= bytes + kMultipoleSumMargin;
+    return fr + buf.cap >= bytes + margin;
+}
+
+bool multipole_buffer_fits(const DevBuf &buf, size_t bytes) {
+    return bytes <= kMultipoleSumBudget && buffer_fits(buf, bytes, kMultipoleSumMargin);
 }
 
 // Atom ranges of a multipole call, each of which rounds its amplitudes to
@@ -495,32 +503,37 @@ int run_batch(sx_ctx *c, int ns, size_t NM, const double *qv, const double *qlen
         // few frames: one orientation a lane (no trials of tile shapes, which
         // run the other form)
         bool few = oriented && !mp && !c->noalloc && sx::few_frames(NF, c->NFp, (int)NM);
-        if (few && c->cfg.tile_shape == 0) {
-            shape = default_shape(c, ns, b_shell != nullptr);
-        } else if (oriented && !mp) {
-            int rc = pick_shape(c, ns, (int)NM, bptr, b_shell != nullptr, &shape);
-            if (rc != SX_OK) return rc;
-        }
-        int split = 1;
+        const size_t pack_bytes = sizeof(float4) * c->NAp * NF;
+        size_t few_bytes = 0;
+        int split = 1, sub = 1;
         if (!oriented && !mp) {
             int rc = pick_all_split(c, V, vb, browp != nullptr, &split);
             if (rc != SX_OK) return rc;
         }
-        if (oriented && !mp) {
+        while (oriented && !mp) {
+            if (few && c->cfg.tile_shape == 0) {
+                shape = default_shape(c, ns, b_shell != nullptr);
+            } else {
+                int rc = pick_shape(c, ns, (int)NM, bptr, b_shell != nullptr, &shape);
+                if (rc != SX_OK) return rc;
+            }
             int rc = pick_oriented_split(c, sx::oriented_base_blocks(c->NFp, (int)NM, ns, shape), shape,
                                          b_shell != nullptr, c->q_mode, (size_t)ns * NM, &split);
             if (rc != SX_OK) return rc;
+            if (!few) break;
+            // with memory for the packed atoms and the parts, beside the amplitudes of one range
+            sub = sx::few_parts(NF, c->NAp, (int)NM, ns, split, shape);
+            few_bytes = pack_bytes + sizeof(double2) * (size_t)V * NF * split * sub;
+            if (few_bytes <= kAmpBudgetBytes &&
+                buffer_fits(c->few, few_bytes, kFewMargin + sizeof(float2) * (size_t)V * c->NFp))
+                break;
+            few = false;
         }
         if (mp) {
             int rc = pick_multipole_split(c, mp->kind, ns, (int)NM, &split);
             if (rc != SX_OK) return rc;
         }
         const size_t split_stride = (size_t)V * c->NFp;
-        int sub = 1;
-        if (few) {
-            sub = sx::few_parts(NF, c->NAp, (int)NM, ns, split, shape);
-            few = sizeof(double2) * (size_t)V * NF * split * sub <= kAmpBudgetBytes;
-        }
         SX_HIP(c, c->amp.ensure(sizeof(float2) * split_stride * (few ? 1 : split)));
         if (mp) {
             SX_HIP(c, c->mpmom.ensure(sizeof(int) * mp->moments.size()));
@@ -629,9 +642,9 @@ int run_batch(sx_ctx *c, int ns, size_t NM, const double *qv, const double *qlen
             int urc = upload_tile_lines(c, ns, shape, &plain);
             if (urc != SX_OK) return urc;
             if (few) {
-                SX_HIP(c, c->pack.ensure(sizeof(float4) * c->NAp * NF));
-                SX_HIP(c, c->fparts.ensure(sizeof(double2) * (size_t)V * NF * split * sub));
-                SX_HIP(c, sx::launch_amp_few(oa, NF, sub, c->pack.as<float4>(), c->fparts.as<double2>(), c->stream));
+                SX_HIP(c, c->few.ensure(few_bytes));
+                double2 *parts = reinterpret_cast<double2 *>(static_cast<char *>(c->few.p) + pack_bytes);
+                SX_HIP(c, sx::launch_amp_few(oa, NF, sub, c->few.as<float4>(), parts, c->stream));
                 split = 1;  // the ranges are added
             } else {
                 SX_HIP(c, sx::launch_amp_oriented(oa, c->stream));
@@ -927,7 +940,7 @@ void sx_destroy(sx_ctx *c) {
     if (!c) return;
     (void)hipSetDevice(c->cfg.device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
-    for (DevBuf *d : {&c->coords, &c->b, &c->twL, &c->twL64, &c->twp, &c->twp64, &c->tw64, &c->w, &c->aidx, &c->apair, &c->tail, &c->qrev, &c->qlen, &c->uvec, &c->brow, &c->bshell, &c->mpmom, &c->mpq, &c->mpsph, &c->mpj, &c->mptab, &c->mpsum, &c->qres, &c->redbuf, &c->pack, &c->fparts, &c->amp,
+    for (DevBuf *d : {&c->coords, &c->b, &c->twL, &c->twL64, &c->twp, &c->twp64, &c->tw64, &c->w, &c->aidx, &c->apair, &c->tail, &c->qrev, &c->qlen, &c->uvec, &c->brow, &c->bshell, &c->mpmom, &c->mpq, &c->mpsph, &c->mpj, &c->mptab, &c->mpsum, &c->qres, &c->redbuf, &c->few, &c->amp,
                       &c->ppart, &c->apart, &c->fqt, &c->fq, &c->fq2, &c->stage, &c->stage2})
         d->release();
     for (auto &e : c->ev)
@@ -1085,6 +1098,10 @@ int sx_stage(sx_ctx *c, const float *xyz, size_t NA, size_t NF, int layout) {
     size_t free_b = 0, total_b = 0;
     SX_HIP(c, hipMemGetInfo(&free_b, &total_b));
     const size_t need = (block > c->coords.cap ? block - c->coords.cap : 0) + ((size_t)64 << 20);
+    if (need > free_b && c->few.p) {
+        c->few.release();  // the last block's packed atoms
+        SX_HIP(c, hipMemGetInfo(&free_b, &total_b));
+    }
     if (need > free_b)
         return fail(c, SX_ERR_NOMEM,
                     "sx_stage: %zu atoms x %zu frames need %zu bytes of device memory, %zu of %zu are free", NA, NF,

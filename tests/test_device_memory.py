@@ -65,3 +65,43 @@ for room in range(full // MB + 8, 120, -8):
 assert grids == sorted(grids, reverse=True), grids
 assert grids[0] // grids[-1] == 17 and len(set(grids)) == 5, grids   # 17, 8, 4, 2, 1 parts
 """)
+
+
+FEW = SETUP + """
+q, u = np.linspace(0.3, 3.0, 40), units(500)
+def call(dev, q=q, u=u):
+    launches()
+    dev.compute_oriented(q, u)
+    return launches()
+"""
+
+
+def test_few_frames_without_room_for_the_packed_atoms(fake_run):  # noqa: F811
+    """40 frames: the packed copy and its parts would not fit beside the staged
+    block; the kernel of a frame a lane runs as it did."""
+    fake_run(FEW + """
+fake.fake_memory(8 * GB)
+dev = staged(200000, 40, dsp="square")
+assert ran(call(dev, q[:4]), "amp_few")
+dev.close()
+dev = staged(200000, 40, dsp="square")
+fake.fake_memory(fake.fake_used() + 100 * (1 << 20))
+names = call(dev, q[:4])
+assert ran(names, "amp_direct") or ran(names, "amp_oriented"), names
+assert not ran(names, "amp_few")
+""")
+
+
+def test_stage_reuses_the_memory_of_packed_atoms(fake_run):  # noqa: F811
+    """A larger block than before where only the packed copy stands in the way."""
+    fake_run(FEW + """
+fake.fake_memory(8 * GB)
+dev = staged(200000, 40, dsp="square")
+assert ran(call(dev, q[:4]), "amp_few")
+# the block grows by 100,000 atoms x 64 frames x 12 B; most of it is in the copy (128 MB)
+fake.fake_memory(fake.fake_used() + 100 * (1 << 20))
+dev.stage(np.zeros((3, 300000, 40), np.float32))
+dev.set_factors(np.ones(300000))
+fake.fake_memory(16 * GB)
+assert ran(call(dev, q[:4]), "amp_few")
+""")
