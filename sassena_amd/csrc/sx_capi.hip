@@ -416,7 +416,12 @@ int run_batch(sx_ctx *c, int ns, size_t NM, const double *qv, const double *qlen
     // general-vector amplitude kernel and the self kernels; the coherent
     // oriented kernel forms q from |q| and the orientations
     const bool need_qrev = mp == nullptr && (!oriented || self);
-    std::vector<double> qh(need_qrev ? 3 * (size_t)V : 0);
+    // the host tables of the call: copies are queued from them, so that they live
+    // until the stream is synchronised at the end
+    std::vector<double> qh(need_qrev ? 3 * (size_t)V : 0), ql;
+    std::vector<float> bs;
+    std::vector<int> br;
+    std::vector<char> tables;
     if (need_qrev && qv) {
         for (size_t i = 0; i < qh.size(); ++i) qh[i] = qv[i] / kTwoPi;
     } else if (need_qrev) {
@@ -425,7 +430,7 @@ int run_batch(sx_ctx *c, int ns, size_t NM, const double *qv, const double *qlen
                 for (int k = 0; k < 3; ++k) qh[(s * NM + m) * 3 + k] = qlen[s] * u[3 * m + k] / kTwoPi;
     }
     if (oriented) {
-        std::vector<double> ql(ns);
+        ql.resize(ns);
         for (int s = 0; s < ns; ++s) ql[s] = qlen[s] / kTwoPi;
         sx::ShellGrid g;
         c->q_mode = sx::shell_progression(ql.data(), ns, c->rmax, &g);
@@ -455,7 +460,7 @@ int run_batch(sx_ctx *c, int ns, size_t NM, const double *qv, const double *qlen
         // rows of atoms per shell; the oriented coherent kernel reads the
         // shells' factors of an atom together
         const bool by_atom = oriented && !self;
-        std::vector<float> bs((size_t)ns * c->NAp + (by_atom ? sx::kShellFactorPad : 0), 0.f);
+        bs.assign((size_t)ns * c->NAp + (by_atom ? sx::kShellFactorPad : 0), 0.f);
         if (by_atom) {
             for (size_t j0 = 0; j0 < c->NA; j0 += 16)
                 for (int s = 0; s < ns; ++s)
@@ -471,7 +476,7 @@ int run_batch(sx_ctx *c, int ns, size_t NM, const double *qv, const double *qlen
                                  c->stream));
         bptr = c->bshell.as<float>();
         if (!self && !by_atom) {
-            std::vector<int> br(V);
+            br.resize(V);
             for (int v = 0; v < V; ++v) br[v] = v / (int)NM;
             SX_HIP(c, c->brow.ensure(sizeof(int) * V));
             SX_HIP(c, hipMemcpyAsync(c->brow.p, br.data(), sizeof(int) * V, hipMemcpyHostToDevice, c->stream));
@@ -617,7 +622,7 @@ int run_batch(sx_ctx *c, int ns, size_t NM, const double *qv, const double *qlen
                 if (sub > 0) {
                     SX_HIP(c, c->mpsum.ensure(part_bytes(sub) + angle_bytes));
                     if (mp->kind == 0) {
-                        std::vector<char> tables(sx::sphere_table_bytes(sp));
+                        tables.resize(sx::sphere_table_bytes(sp));
                         sx::sphere_tables(sp, tables.data());
                         SX_HIP(c, c->mptab.ensure(tables.size()));
                         SX_HIP(c, hipMemcpyAsync(c->mptab.p, tables.data(), tables.size(), hipMemcpyHostToDevice,
