@@ -11,7 +11,7 @@ struct OrientKernelArgs {
     size_t NFp;
     const double *qlen;    // [ns] |q_s| / 2 pi
     const double *u;       // [NM][3] unit orientations
-    const float *b;        // [NAp], or one factor per shell and atom: [NAp][ns] and kWave floats more
+    const float *b;        // [NAp], or one factor per shell and atom: [NAp][ns] and kShellFactorPad floats more
     size_t NAp;            // row stride of the coordinate planes
     size_t natoms;         // atoms summed (<= NAp)
     int NM, ns, V, ftiles, ogroups, sgroups, split, atoms_per_split, per_shell_b;
@@ -94,6 +94,7 @@ __device__ __forceinline__ void oriented_tile_body(const OrientKernelArgs &a, in
     constexpr bool RES = UPC || DNC;
     static_assert(!(LT && PER_ROW_B), "residual-corrected tiles take one factor per atom");
     static_assert(!LQ || VM == 1, "one orientation a lane");
+    static_assert(VS - 1 <= (int)kShellFactorPad, "the last atom's factors are read for VS shells");
     constexpr int CH = LQ ? 8 : 16;  // atoms per coordinate batch
     constexpr int kFold = 64;  // atoms per FP32 partial sum
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);

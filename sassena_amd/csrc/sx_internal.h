@@ -112,6 +112,8 @@ struct TileLine {
 };
 constexpr int kTileCorrectUp = 1, kTileCorrectDown = 2;
 
+// Floats behind the factors per atom and shell: a tile reads those of all its
+// shells, the last tile's past the last shell too.
 constexpr size_t kShellFactorPad = 32;
 
 // Oriented shells: v = s * NM + m has q_v = |q_s| u_m.  NAp must be a multiple
