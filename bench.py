@@ -57,12 +57,11 @@ AMP_TRAFFIC_BYTES = 2.467e9 + 0.524e9
 # FP64 flops per (atom, frame, moment, shell) term of the multipole amplitude
 # kernels on the mp / mpc workloads: rocprofv3 counts of FP64 FMA (2 flops),
 # MUL and ADD wave instructions x 64 lanes over the terms of one launch
-# (sphere 4.84e10 terms, cylinder 1.64e10), plus those of the pre-pass that
-# tabulates the Bessel functions of every (shell, atom, frame), both inside
-# the timed multipole stage: sphere 18.9 + 1.1 (0.92e12 + 0.05e12 flops),
-# cylinder 27.9 + 15.5 (0.46e12 + 0.25e12; the cylinder's pre-pass also
-# forms the two phases e^{i sgn z q_z} and e^{i psi}).
-MP_FP64_PER_TERM = {"sphere": 20.0, "cylinder": 43.4}
+# (sphere 4.84e10 terms, cylinder 1.64e10), over the timed multipole stage:
+# sphere 4.67 in the sums and 0.25 in the spherical terms (2.26e11 + 0.12e11
+# flops), cylinder 16.28 in the sums and 0.45 in the cylinder terms, angles and
+# amplitudes (2.67e11 + 0.07e11).
+MP_FP64_PER_TERM = {"sphere": 4.9, "cylinder": 16.7}
 
 
 def roofline_legs(terms_per_launch, launch_s):
@@ -261,9 +260,9 @@ def bench_mp(args):
         amp_s = amp_ms / args.steps * 1e-3
         out["roofline"] = {"bound": "valu", "achieved": per * terms / amp_s / 1e12, "peak": FP64_PEAK / 1e12,
                            "unit": "TFLOP/s", "frac": per * terms / amp_s / FP64_PEAK, "traffic": None,
-                           "kernel": "multipole_kernel", "fp64_flops_per_term": per,
+                           "kernel": f"{kind}_sums_kernel", "fp64_flops_per_term": per,
                            "note": "FP64 flops per (atom, frame, moment, shell) from rocprofv3 counts of "
-                                   "FP64 FMA (2 flops), MUL and ADD instructions over the multipole kernel, "
+                                   "FP64 FMA (2 flops), MUL and ADD instructions over the multipole stage, "
                                    "against the published FP64 vector peak"}
     if not args.no_cpu:
         # the FP64 oracle on the host: one shell x one moment per thread

@@ -211,7 +211,7 @@ constexpr size_t kStageKeepBytes = (size_t)16 << 20;
 constexpr size_t kSplitBudgetBytes = (size_t)16 << 30;
 
 // The FFT plan and tables of the staged number of frames, which alone they depend
-// on: kept from one block to the next of as many frames (host sines, six
+// on: kept from one block to the next of as many frames (host sines, five
 // copies and the weights: 1,000 atoms x 200 frames staged and scanned at 10 shells x
 // 50 vectors 490 -> 374 us with this and the transpose buffer kept).
 int prepare_tables(sx_ctx *c) {

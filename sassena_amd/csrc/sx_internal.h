@@ -126,7 +126,7 @@ struct OrientArgs {
     // [NAp], or if per_shell_b [NAp][ns] with kShellFactorPad floats behind (the
     // factors of a tile's shells are then one scalar load an atom; as rows of
     // atoms they took the scalar registers of 16 atoms x 8 shells: 9.1 ms against
-    // 4.7 for 7,001 atoms x 1,501 frames x 21 shells x 67 orientations)
+    // 4.9, both in tiles of 8 shells, for 7,001 atoms x 1,501 frames x 21 shells x 67 orientations)
     const float *b;
     int NM, ns, split, per_shell_b;
     int shape = 0;         // tile shape index (< kOrientShapes)

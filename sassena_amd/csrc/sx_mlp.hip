@@ -27,7 +27,7 @@
 // workgroups follow in order.  Products that enter a sum do so by fmaf, which
 // leaves the compiler no choice of which one to fuse.  (Adam carries a rounding
 // of one sum into the fourth digit of the parameters within 500 steps.)
-// 4,096 rows a step: 14 + 5 us (133 + 16 us when each of four wavefronts took 16
+// 4,096 rows a step: 14 + 4 us (133 + 16 us when each of four wavefronts took 16
 // rows through all columns, copied W2 into LDS and added its gradients there
 // by LDS atomics).
 #include <hip/hip_runtime.h>

@@ -15,8 +15,8 @@
 // Bound by FP64 issue and the latency of its chains: per (atom, frame, shell)
 // about 10 operations an order and 130 to 180 for the first two functions or
 // Miller's recurrence; the sums of 21 orders leave two wavefronts a SIMD.
-// 10,000 atoms x 2,000 frames, 41 moments, 10 shells: 6.8 ms (45 ms when a
-// pre-pass stored J_n of every (shell, order, atom, frame), 34 GB here, and each
+// 10,000 atoms x 2,000 frames, 41 moments, 10 shells: 6.8 ms, 7.2 ms a call (45 ms a
+// call when a pre-pass stored J_n of every (shell, order, atom, frame), 34 GB here, and each
 // wavefront of 8 moments formed its own phases).
 #include <algorithm>
 #include <cmath>

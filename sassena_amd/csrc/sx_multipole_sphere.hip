@@ -23,9 +23,9 @@
 // functions of a shell; at most 100 sums a lane, so that two wavefronts a SIMD
 // fit without scratch.  Bound by the latency of those two (scalar and LDS loads
 // per entry, the recurrences of the factors).  20,000 atoms x 2,000 frames,
-// 121 moments, 10 shells: 15.8 ms (128 ms when each wavefront of 8 moments ran
-// their Legendre recurrences itself and read Bessel functions from a table of
-// 36 GB); no call of its degrees was faster that way.
+// 121 moments, 10 shells: 15.8 ms, 16.5 ms a call (128 ms a call when each wavefront
+// of 8 moments ran their Legendre recurrences itself and read Bessel functions
+// from a table of 36 GB).
 #include <algorithm>
 #include <cmath>
 
